@@ -21,6 +21,7 @@
 //    over query_start_loc), so a call needs no host copy of the batch layout.
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -505,9 +506,20 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
 //     and lo = RN(p - hi): both products with a value are exact in float32, so the sum carries p
 //     to about 2^-17 relative, the float32 arithmetic of the reference's kernel (a single 16-bit
 //     P would round each weight by up to 2^-9).
-// The scores are the float32 dot products times scale * log2(e) and exp2 replaces exp, as in the
-// decode kernel.  A tile whose positions span several partitions has them merged by the last to
-// arrive, as the decode kernel's split rows are.
+// The scores are the float32 dot products times scale * log2(e) (folded into the exponent's fma)
+// and exp2 replaces exp, as in the decode kernel.
+//
+// Work split: all steps of all (tile, KV head) pairs are shared evenly by up to 512 workgroups (two
+// per CU, all resident), each taking a run of consecutive steps, so that they end together whatever
+// the sequences' lengths and a tile is cut only where a run ends: at most two partials per
+// workgroup, stored and merged in the lanes' accumulator layout (256 contiguous bytes per 4-byte
+// element of a wave).  Four 512-token chunks ending at 2048 .. 8192 positions (24 / 8 heads of 128
+// dims, bf16): 627 -> 257 us, 195 -> 475 TFLOP/s, against partitions of at most 1024 positions whose
+// 64 KB of partials each went out and came back as scattered 4-byte accesses; three chunks of up to
+// 417 tokens beside 29 decode rows (32 / 8 heads of 64 dims, f16): 89 -> 55 us for the call.
+// Keys and values are double buffered in LDS (one barrier a step), the value rows at a pitch under
+// which a transposing read's four rows hit different banks (the key rows' pitch left them 4-way
+// conflicted), and the block table is read one step ahead of the rows instead of through LDS.
 
 constexpr int kPfWaves = 4;
 constexpr int kPfThreads = 64 * kPfWaves;
@@ -516,6 +528,7 @@ constexpr int kPfPos = 64;               // positions per step (two 32-row block
 constexpr int kPfMaxPart = 1024;
 constexpr int kPfMinPart = 256;
 constexpr int kPfTargetGroups = 512;     // two four-wave workgroups per CU
+constexpr int kPfMinSteps = 4;           // steps a workgroup takes at least when tiles are cut
 static_assert(kPfCols == NS_PA_TILE_COLUMNS, "the header's tile width");
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -557,12 +570,57 @@ template <> struct Mma<F16> {
 
 struct PfParams {
   const int32_t* tiles;   // (n_tiles, 3): sequence, first query token (flat index), token count
-  float* ws_acc;          // (n_tiles, hkv, max_parts, kPfCols, D) unnormalised partition outputs
-  float* ws_ml;           // (n_tiles, hkv, max_parts, kPfCols, 2) partition max (log2 units), sum
-  int32_t* counters;      // (n_tiles, hkv) arrivals of split tiles; zero between calls
-  int32_t part_tokens;    // positions per partition (a multiple of kPfPos)
-  int32_t max_parts;      // at least 1
+  float* ws_acc;          // (slots, kPfWaves, D / 2, 64 lanes) unnormalised outputs of cut tiles, as the lanes hold them
+  float* ws_ml;           // (slots, kPfCols, 2) their max (log2 units) and sum
+  int32_t* counters;      // (n_tiles, hkv) arrivals of a cut tile's segments; zero between calls
+  int32_t n_tiles;
+  int32_t grid;           // workgroups that share all steps evenly, or 0: one workgroup per (tile, KV head)
+  int64_t cap;            // positions of a sequence the call takes (max_seq_len, rounded up to a partition)
+  float scale_log2;       // |scale| * log2(e); 1 for a scale of 0
+  uint32_t q_and, q_xor;  // applied to the query words: a negative scale flips their signs, a zero scale clears them
+  int32_t out_vec;        // output rows 8-byte aligned: four elements a store
 };
+
+struct PfTile {
+  int seq, t0, nq;
+  int kv_pos0;   // the first token's KV position
+  int lt;        // positions the last token sees, up to the call's capacity
+  int steps;     // 64-position steps (at least 1), or 0: not a tile of this batch
+  bool cut;      // the sequence is longer than the capacity
+};
+
+__device__ __forceinline__ PfTile pf_tile(const PaParams& p, const PfParams& f, int tile, int bq) {
+  PfTile r;
+  r.seq = f.tiles[3 * tile];
+  r.t0 = f.tiles[3 * tile + 1];
+  r.nq = f.tiles[3 * tile + 2];
+  r.steps = 0;
+  r.kv_pos0 = r.lt = 0;
+  r.cut = false;
+  // a tile must hold 1 .. bq consecutive query tokens of one sequence: anything else is flagged
+  // and left alone (nothing is read or written out of bounds)
+  if (r.seq < 0 || r.seq >= p.num_seqs || r.nq < 1 || r.nq > bq || r.t0 < 0) return r;
+  const int q0 = p.qsl[r.seq], ql = p.qlens[r.seq];
+  if (r.t0 < q0 || (int64_t)r.t0 + r.nq > (int64_t)q0 + ql || (int64_t)r.t0 + r.nq > p.total_q) return r;
+  const int seq_len = p.seq_lens[r.seq];
+  r.kv_pos0 = seq_len - ql + (r.t0 - q0);
+  int lt = r.kv_pos0 + r.nq < seq_len ? r.kv_pos0 + r.nq : seq_len;
+  if (lt < 0) lt = 0;
+  r.cut = lt > f.cap;
+  r.lt = r.cut ? (int)f.cap : lt;
+  r.steps = r.lt > 0 ? (r.lt + kPfPos - 1) / kPfPos : 1;
+  return r;
+}
+
+__device__ __forceinline__ void st_dev2(float* p, float a, float b) {
+  const uint64_t w = (uint64_t)__float_as_uint(a) | ((uint64_t)__float_as_uint(b) << 32);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x2 ld_dev2(const float* p) {
+  const uint64_t w = __hip_atomic_load(reinterpret_cast<uint64_t*>(const_cast<float*>(p)), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+  return f32x2{__uint_as_float((uint32_t)w), __uint_as_float((uint32_t)(w >> 32))};
+}
 
 template <typename T, int D, int G>
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void pa_prefill_kernel(PaParams p,
@@ -574,354 +632,405 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
   constexpr int DB = D / 32;                      // 32-dim blocks of O^T
   constexpr int CPP = D / 8;                      // 16-byte chunks of a key or value row
   constexpr int LPT = kPfPos * CPP / kPfThreads;  // chunks of each kind a thread loads per step
-  constexpr int PK = D * 2 + 16;                  // bytes per staged key or value row
+  // bytes per staged row: keys so that 16 rows' 16-byte reads hit the 64 banks once, values so
+  // that the four rows of a transposing read do
+  constexpr int PK = D * 2 + 16;
+  constexpr int PV = D * 2 + 64;
   static_assert(LPT * kPfThreads == kPfPos * CPP, "the step's chunks split evenly over the threads");
-  __shared__ __align__(16) unsigned char s_k[kPfPos * PK];
-  __shared__ __align__(16) unsigned char s_v[kPfPos * PK];
-  __shared__ __align__(16) uint8_t s_ok[kPfPos];
-  __shared__ int s_blk[kPfMaxPart + 2];
+  __shared__ __align__(16) unsigned char s_k[2][kPfPos * PK];
+  __shared__ __align__(16) unsigned char s_v[2][kPfPos * PV];
+  __shared__ int64_t s_wave[kPfWaves];
+  __shared__ int s_place[2];   // the workgroup's first tile and its step in it
+  __shared__ int s_bad;        // an invalid block met in this segment
   __shared__ int s_last;
 
-  const int tile = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, c32 = lane & 31;
-  const int seq = f.tiles[3 * tile];
-  const int t0 = f.tiles[3 * tile + 1];
-  const int nq = f.tiles[3 * tile + 2];
-  // a tile must hold 1 .. BQ consecutive query tokens of one sequence: anything else is flagged
-  // and left alone (nothing is read or written out of bounds)
-  if (seq < 0 || seq >= p.num_seqs || nq < 1 || nq > BQ || t0 < p.qsl[seq] || t0 + nq > p.qsl[seq] + p.qlens[seq] ||
-      t0 + nq > p.total_q) {
-    if (tid == 0 && part == 0 && p.status) atomicOr(p.status, NS_PA_STATUS_BAD_TILE);
-    return;
-  }
-  const int seq_len = p.seq_lens[seq];
-  const int kv_pos0 = seq_len - p.qlens[seq] + (t0 - p.qsl[seq]);   // the first token's KV position
-  int lt = kv_pos0 + nq < seq_len ? kv_pos0 + nq : seq_len;          // positions the last token sees
-  if (lt < 0) lt = 0;
-  const int n_parts = (lt + f.part_tokens - 1) / f.part_tokens;
-  if (part == 0 && n_parts > f.max_parts && tid == 0 && p.status) atomicOr(p.status, NS_PA_STATUS_SEQ_TOO_LONG);
+  const int n_tiles = f.n_tiles;
 
-  // the lane's column: token tok, head hd, visible positions kvl (-1: a padding column, never written)
-  const int c = wave * 32 + c32;
-  const int tok = c / G, hd = c % G;
-  int kvl = -1;
-  if (c < BQ * G && tok < nq) {
-    const int kl = kv_pos0 + tok + 1 < seq_len ? kv_pos0 + tok + 1 : seq_len;
-    kvl = kl > 0 ? kl : 0;
-  }
-  const int64_t obase = (int64_t)(t0 + tok) * p.so_tok + (int64_t)(kvh * G + hd) * p.so_head;
-  if (part >= n_parts) {
-    if (part == 0 && kvl >= 0 && h == 0)   // no visible key for any token of the tile: zeros
-      for (int d = 0; d < D; ++d) store_one<T>(p.out, obase + d, 0.f);
-    return;
-  }
-  const int j0 = part * f.part_tokens;
-  const int j1 = lt < j0 + f.part_tokens ? lt : j0 + f.part_tokens;
-  const int kend = kvl < j1 ? kvl : j1;   // the column's positions below kend are visible here
-  // the smallest kend of the wave's columns (padding columns aside): positions below it are
-  // visible to every column of the wave
-  int kend_w = kvl >= 0 ? kend : INT32_MAX;
-#pragma unroll
-  for (int sh = 1; sh < 64; sh <<= 1) kend_w = min(kend_w, __shfl_xor(kend_w, sh));
-  const int32_t* bt_row = p.bt + (int64_t)seq * p.sbt;
-  // the partition's slice of the block table, validated once, into LDS
-  const int bi0 = j0 / p.block_size;
-  const int nbi = (j1 - 1) / p.block_size - bi0 + 1;
-  int bad = 0;
-  for (int i = tid; i < nbi; i += kPfThreads) {
-    const int bi = bi0 + i;
-    int blk = bi < p.max_blocks_per_seq ? bt_row[bi] : -1;
-    if (blk < 0 || blk >= p.num_blocks) {
-      blk = -1;
-      bad = 1;
-      if (p.status) atomicOr(p.status, NS_PA_STATUS_BAD_BLOCK);
+  // The workgroup's units: unit u of all hkv * S steps is step u % S of the tiles in order, KV
+  // head u / S.  Each workgroup takes `per` consecutive units, so that all of them finish
+  // together whatever the sequences' lengths; a tile cut between workgroups is merged by the
+  // last of them to arrive.
+  int64_t u0 = 0, u1 = 0, per = 1, S = 0;
+  int w = 0, tile = 0, off = 0, kvh = 0;
+  if (f.grid > 0) {
+    const int q = (n_tiles + kPfThreads - 1) / kPfThreads;   // tiles per thread, consecutive
+    const int first = tid * q;
+    int64_t mine = 0;
+    for (int i = first; i < first + q && i < n_tiles; ++i) {
+      const PfTile t = pf_tile(p, f, i, BQ);
+      mine += t.steps;
+      if (blockIdx.x == 0 && p.status) {
+        if (t.steps == 0) atomicOr(p.status, NS_PA_STATUS_BAD_TILE);
+        if (t.cut) atomicOr(p.status, NS_PA_STATUS_SEQ_TOO_LONG);
+      }
     }
-    s_blk[i] = blk;
-  }
-
-  // Q^T operand: column c, dims 16 ks + 8 h .. + 7 (zeros for a padding column)
-  vec qop[KS];
-  {
-    const int64_t qoff = (int64_t)(t0 + tok) * p.sq_tok + (int64_t)(kvh * G + hd) * p.sq_head;
+    int64_t pre = mine;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      u32x4 w = {0u, 0u, 0u, 0u};
-      if (kvl >= 0) w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(p.q) + (qoff + 16 * ks + 8 * h) * 2);
-      qop[ks] = __builtin_bit_cast(vec, w);
+    for (int sh = 1; sh < 64; sh <<= 1) {
+      const int64_t o = __shfl_up(pre, sh);
+      if (lane >= sh) pre += o;
     }
+    if (lane == 63) s_wave[wave] = pre;
+    __syncthreads();
+    for (int i = 0; i < kPfWaves; ++i) {
+      if (i < wave) pre += s_wave[i];
+      S += s_wave[i];
+    }
+    pre -= mine;
+    const int64_t U = S * p.hkv;
+    per = (U + f.grid - 1) / f.grid;
+    if (per < kPfMinSteps) per = kPfMinSteps;
+    w = blockIdx.x;
+    u0 = per * w;
+    u1 = u0 + per < U ? u0 + per : U;
+    if (u0 >= U) return;
+    kvh = (int)(u0 / S);
+    const int64_t rem = u0 - kvh * S;
+    if (rem >= pre && rem < pre + mine) {
+      int64_t at = rem - pre;
+      int i = first;
+      for (;; ++i) {   // the thread's steps hold `at`: one of its tiles does
+        const int n = pf_tile(p, f, i, BQ).steps;
+        if (at < n) break;
+        at -= n;
+      }
+      s_place[0] = i;
+      s_place[1] = (int)at;
+    }
+    __syncthreads();
+    tile = s_place[0];
+    off = s_place[1];
+  } else {
+    tile = blockIdx.x % n_tiles;
+    kvh = blockIdx.x / n_tiles;
+    const PfTile t = pf_tile(p, f, tile, BQ);
+    if (tid == 0 && kvh == 0 && p.status) {
+      if (t.steps == 0) atomicOr(p.status, NS_PA_STATUS_BAD_TILE);
+      if (t.cut) atomicOr(p.status, NS_PA_STATUS_SEQ_TOO_LONG);
+    }
+    if (t.steps == 0) return;
+    u1 = t.steps;
   }
-  // the slice, and whether any of its blocks is invalid (then every step masks by position)
-  const bool any_bad = __syncthreads_or(bad) != 0;
 
-  // the step's key and value rows: chunk i = tid + kPfThreads r is position i / CPP, dims
-  // 8 (i % CPP) .. + 7; zeros past the partition or for an invalid block
-  // every chunk of the thread has dims 8 dc .. (kPfThreads is a multiple of CPP); the host
+  // every chunk of the thread has dims 8 dc .. + 7 (kPfThreads is a multiple of CPP); the host
   // keeps token strides times block_size below 2^31, so a slot's offset is a 32-bit product
   const int dc0 = tid % CPP;
-  const char* kbase = reinterpret_cast<const char*>(p.k) + ((int64_t)kvh * p.sk_head + 8 * dc0) * 2;
-  const char* vbase = reinterpret_cast<const char*>(p.v) + ((int64_t)kvh * p.sv_head + 8 * dc0) * 2;
   const int sk_tok = (int)p.sk_tok, sv_tok = (int)p.sv_tok;
-  auto load_step = [&](int jt, u32x4 (&kreg)[LPT], u32x4 (&vreg)[LPT], bool (&okr)[LPT]) {
-#pragma unroll
-    for (int r = 0; r < LPT; ++r) {
-      const int j = jt + (tid + kPfThreads * r) / CPP;
-      int blk = -1, off = 0;
-      if (j < j1) {
-        int bi;
-        if (p.bs_shift >= 0) { bi = j >> p.bs_shift; off = j & (p.block_size - 1); }
-        else { bi = j / p.block_size; off = j - bi * p.block_size; }
-        blk = s_blk[bi - bi0];
-      }
-      okr[r] = blk >= 0;
-      kreg[r] = u32x4{0u, 0u, 0u, 0u};
-      vreg[r] = u32x4{0u, 0u, 0u, 0u};
-      if (blk >= 0) {
-        kreg[r] = *reinterpret_cast<const u32x4*>(kbase + ((int64_t)blk * p.sk_blk + off * sk_tok) * 2);
-        vreg[r] = *reinterpret_cast<const u32x4*>(vbase + ((int64_t)blk * p.sv_blk + off * sv_tok) * 2);
-      }
-    }
-  };
-  auto store_step = [&](const u32x4 (&kreg)[LPT], const u32x4 (&vreg)[LPT], const bool (&okr)[LPT]) {
-#pragma unroll
-    for (int r = 0; r < LPT; ++r) {
-      const int i = tid + kPfThreads * r;
-      const int pos = i / CPP, dc = i % CPP;
-      *reinterpret_cast<u32x4*>(s_k + pos * PK + dc * 16) = kreg[r];
-      *reinterpret_cast<u32x4*>(s_v + pos * PK + dc * 16) = vreg[r];
-      if (dc == 0) s_ok[pos] = okr[r] ? 1 : 0;
-    }
-  };
-
-  f32x16_t acc[DB];
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
-  float m = -INFINITY, l = 0.f;
-
   // The transposing read (ds_read_b64_tr_b16): in each 16-lane group, lane j's four results are
   // element j % 4 of the 4-element rows that lanes 4 m + j / 4 address, m = 0..3.  So that lane L
   // receives positions 16 s + 4 h + m of dim 32 db + L % 32, lane L addresses position
   // 16 s + 4 (L / 32) + (L % 16) / 4, dims 32 db + 16 ((L / 16) % 2) + 4 (L % 4) .. + 3.
   const int tr_pos = 4 * (lane >> 5) + ((lane & 15) >> 2);
   const int tr_dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  u32x4 kreg[LPT], vreg[LPT];
-  bool okr[LPT];
-  load_step(j0, kreg, vreg, okr);
-  for (int jt = j0; jt < j1; jt += kPfPos) {
-    __syncthreads();   // the previous step's reads of the staged rows are done
-    store_step(kreg, vreg, okr);
-    __syncthreads();   // this step's rows staged
-    // the next step's rows, in flight across this step's products and softmax
-    if (jt + kPfPos < j1) load_step(jt + kPfPos, kreg, vreg, okr);
-    // S^T = K Q^T for the step's two 32-position row blocks (two independent MFMA chains)
-    f32x16_t st[2];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) st[rb][e] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(s_k + (32 * rb + c32) * PK + (16 * ks + 8 * h) * 2);
-        st[rb] = M::mma(__builtin_bit_cast(vec, w), qop[ks], st[rb]);
-      }
-    }
-    // the online softmax of the lane's column over the step's 64 positions (element e of block
-    // rb: position 32 rb + 8 (e / 4) + 4 h + e % 4; the other half in lane ^ 32)
-    float mt = -INFINITY;
-    if (jt + kPfPos <= kend_w && !any_bad) {   // every position of the step visible to every column
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          st[rb][e] *= p.scale_log2;
-          mt = fmaxf(mt, st[rb][e]);
-        }
-    } else {
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        uint32_t okw[4] = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};
-        if (any_bad) {
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) okw[q4] = *reinterpret_cast<const uint32_t*>(s_ok + 32 * rb + 8 * q4 + 4 * h);
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int r = 32 * rb + 8 * (e >> 2) + 4 * h + (e & 3);
-          const bool ok = jt + r < kend && ((okw[e >> 2] >> (8 * (e & 3))) & 0xffu) != 0u;
-          st[rb][e] = ok ? st[rb][e] * p.scale_log2 : -INFINITY;
-          mt = fmaxf(mt, st[rb][e]);
-        }
-      }
-    }
-    mt = fmaxf(mt, __shfl_xor(mt, 32));
-    // The column's reference m moves only when a score exceeds it by more than 8 (log2 units),
-    // to the new maximum: weights stay at most 2^8 and the accumulators are rescaled rarely.
-    // exp2 by v_exp_f32 (a weight below 2^-126 flushes to zero); -inf scores weigh 0, and a
-    // column with no score yet subtracts 0.
-    const bool move = mt > m + 8.f;
-    const float mn = move ? mt : m;
-    const float msub = mn == -INFINITY ? 0.f : mn;
-    const float alpha = move ? __builtin_amdgcn_exp2f(m - msub) : 1.f;
-    m = mn;
-    if (__ballot(move) != 0ull) {   // a column's reference moved: rescale
-      l *= alpha;
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[db][e] *= alpha;
-    }
-    // per 16-position k-step s: P as the hi / lo B operands, then O^T += V^T P^T with the V^T
-    // operand of dim 32 db + c32 (k-slot i of half h at position 16 s + 8 (i / 4) + 4 h + i % 4)
-    // read from the value rows by two transposing reads (k-slots 0-3, then 4-7)
-    float ls = 0.f;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      u32x4 wh, wl;
-#pragma unroll
-      for (int i2 = 0; i2 < 4; ++i2) {
-        const float p0 = __builtin_amdgcn_exp2f(st[s >> 1][8 * (s & 1) + 2 * i2] - msub);
-        const float p1 = __builtin_amdgcn_exp2f(st[s >> 1][8 * (s & 1) + 2 * i2 + 1] - msub);
-        ls += p0 + p1;
-        wh[i2] = M::pack2(p0, p1);
-        wl[i2] = M::pack2(p0 - M::lo(wh[i2]), p1 - M::hi(wh[i2]));
-      }
-      const vec phi = __builtin_bit_cast(vec, wh), plo = __builtin_bit_cast(vec, wl);
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const unsigned char* src = s_v + (16 * s + tr_pos) * PK + (32 * db + tr_dim) * 2;
-        const u32x2 lo4 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                                        (__attribute__((address_space(3))) i16x4*)(src)));
-        const u32x2 hi4 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                                        (__attribute__((address_space(3))) i16x4*)(src + 8 * PK)));
-        const u32x4 w = {lo4[0], lo4[1], hi4[0], hi4[1]};
-        const vec a = __builtin_bit_cast(vec, w);
-        acc[db] = M::mma(a, phi, acc[db]);
-        acc[db] = M::mma(a, plo, acc[db]);
-      }
-    }
-    ls += __shfl_xor(ls, 32);
-    l += ls;
-  }
+  const float scale = f.scale_log2;
+  // the lane's column: token tok, head hd
+  const int c = wave * 32 + c32;
+  const int tok = c / G, hd = c % G;
 
-  // O^T layout: lane l, element e -> column c, dim 32 db + 8 (e / 4) + 4 h + e % 4
-  const bool direct = n_parts == 1;
-  const int64_t wbase = ((int64_t)tile * p.hkv + kvh) * f.max_parts;
-  if ((direct || part < f.max_parts) && kvl >= 0) {
+  for (int64_t u = u0; u < u1;) {
+    if (tile == n_tiles) {
+      tile = 0;
+      ++kvh;
+    }
+    const PfTile t = pf_tile(p, f, tile, BQ);
+    if (t.steps == 0) {   // not a tile of this batch: no units
+      ++tile;
+      continue;
+    }
+    const int take = (int)(u1 - u < t.steps - off ? u1 - u : t.steps - off);
+    // visible positions of the lane's column (-1: a padding column, never written)
+    int kvl = -1;
+    if (c < BQ * G && tok < t.nq) {
+      const int kl = t.kv_pos0 + tok + 1 < t.lt ? t.kv_pos0 + tok + 1 : t.lt;
+      kvl = kl > 0 ? kl : 0;
+    }
+    const bool live = __ballot(kvl >= 0) != 0ull;   // a wave of padding columns only loads rows
+    const int j0 = off * kPfPos;
+    const int j1 = t.lt < j0 + take * kPfPos ? t.lt : j0 + take * kPfPos;
+    const int kend = kvl < j1 ? kvl : j1;   // the column's positions below kend are visible here
+    // the smallest kend of the wave's columns (padding columns aside): positions below it are
+    // visible to every column of the wave
+    int kend_w = kvl >= 0 ? kend : INT32_MAX;
+#pragma unroll
+    for (int sh = 1; sh < 64; sh <<= 1) kend_w = min(kend_w, __shfl_xor(kend_w, sh));
+    const int32_t* bt_row = p.bt + (int64_t)t.seq * p.sbt;
+    const char* kbase = reinterpret_cast<const char*>(p.k) + ((int64_t)kvh * p.sk_head + 8 * dc0) * 2;
+    const char* vbase = reinterpret_cast<const char*>(p.v) + ((int64_t)kvh * p.sv_head + 8 * dc0) * 2;
+
+    // Q^T operand: column c, dims 16 ks + 8 h .. + 7 (zeros for a padding column)
+    vec qop[KS];
+    {
+      const int64_t qoff = (int64_t)(t.t0 + tok) * p.sq_tok + (int64_t)(kvh * G + hd) * p.sq_head;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        u32x4 x = {0u, 0u, 0u, 0u};
+        if (kvl >= 0) x = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(p.q) + (qoff + 16 * ks + 8 * h) * 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = (x[i] & f.q_and) ^ f.q_xor;
+        qop[ks] = __builtin_bit_cast(vec, x);
+      }
+    }
+
+    // Position j's entry of the block table and its offset in the block; the table is read one
+    // step ahead of the rows, the rows one step ahead of the products.  Chunk r of the thread is
+    // position (tid + kPfThreads r) / CPP of a step.
+    auto split = [&](int j, int& o) -> int {
+      int bi;
+      if (p.bs_shift >= 0) { bi = j >> p.bs_shift; o = j & (p.block_size - 1); }
+      else { bi = j / p.block_size; o = j - bi * p.block_size; }
+      return bi;
+    };
+    auto entry = [&](int jt, int r) -> int {   // -1: past the segment or the table
+      const int j = jt + (tid + kPfThreads * r) / CPP;
+      int o;
+      const int bi = split(j < j1 ? j : j1 - 1, o);
+      return j < j1 && bi < p.max_blocks_per_seq ? bt_row[bi] : -1;
+    };
+    u32x4 kreg[LPT], vreg[LPT];
+    int blk[LPT];
+    auto load_entries = [&](int jt) {
+#pragma unroll
+      for (int r = 0; r < LPT; ++r) blk[r] = entry(jt, r);
+    };
+    auto load_rows = [&](int jt, bool (&ok)[LPT]) {
+#pragma unroll
+      for (int r = 0; r < LPT; ++r) {
+        const int j = jt + (tid + kPfThreads * r) / CPP;
+        int o;
+        split(j < j1 ? j : j1 - 1, o);
+        ok[r] = blk[r] >= 0 && blk[r] < p.num_blocks;
+        if (j < j1 && !ok[r]) {
+          s_bad = 1;
+          if (p.status) atomicOr(p.status, NS_PA_STATUS_BAD_BLOCK);
+        }
+        const int b = ok[r] ? blk[r] : 0;   // block 0 stands in for an invalid one; its rows are not used
+        kreg[r] = *reinterpret_cast<const u32x4*>(kbase + ((int64_t)b * p.sk_blk + o * sk_tok) * 2);
+        vreg[r] = *reinterpret_cast<const u32x4*>(vbase + ((int64_t)b * p.sv_blk + o * sv_tok) * 2);
+      }
+    };
+    auto store_rows = [&](int buf, const bool (&ok)[LPT]) {
+#pragma unroll
+      for (int r = 0; r < LPT; ++r) {
+        const int pos = (tid + kPfThreads * r) / CPP;
+        u32x4 x = vreg[r];
+        if (!ok[r]) x = u32x4{0u, 0u, 0u, 0u};   // weight 0 times a row not of this sequence must be 0
+        *reinterpret_cast<u32x4*>(s_k[buf] + pos * PK + dc0 * 16) = kreg[r];
+        *reinterpret_cast<u32x4*>(s_v[buf] + pos * PV + dc0 * 16) = x;
+      }
+    };
+
+    f32x16_t acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int d = 32 * db + 8 * (e >> 2) + 4 * h + (e & 3);
-        if (direct) store_one<T>(p.out, obase + d, l > 0.f ? acc[db][e] / l : 0.f);
-        else st_dev(&f.ws_acc[((wbase + part) * kPfCols + c) * D + d], acc[db][e]);
-      }
-    if (!direct && h == 0) {
-      st_dev(&f.ws_ml[((wbase + part) * kPfCols + c) * 2], m);
-      st_dev(&f.ws_ml[((wbase + part) * kPfCols + c) * 2 + 1], l);
-    }
-  }
-  if (direct || part >= f.max_parts) return;
+      for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
+    float m = -INFINITY, l = 0.f;
 
-  // split tile: the last partition to arrive merges (the partials crossed through agent-scope
-  // atomic stores completed by the s_waitcnt, read back through agent-scope loads)
-  const int arrivals = n_parts < f.max_parts ? n_parts : f.max_parts;
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  int32_t* counter = f.counters + (int64_t)tile * p.hkv + kvh;
-  if (tid == 0) s_last = atomicAdd(counter, 1) == arrivals - 1;
-  __syncthreads();
-  if (!s_last) return;
-  if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // The weights w_i = exp2(m_i - max) of every column's partitions and their sum L: up to
-  // kPfMergeLds partitions in LDS (the staged key rows are free now), computed once, with all
-  // the (m, l) loads of a thread in flight together; then two threads per column, half the dims
-  // each, accumulate the partials partition by partition, all of a partition's loads issued
-  // before the first is used.
-  constexpr int HD = D / 2;
-  constexpr int kPfMergeLds = (kPfPos * PK) / (kPfCols * 4) >= 32 ? 32 : 16;   // partitions in the table
-  float* s_w = reinterpret_cast<float*>(s_k);        // [i][column] weights
-  float* s_L = reinterpret_cast<float*>(s_v);        // [column] the weights' sum of l
-  static_assert(kPfMergeLds * kPfCols * 4 <= kPfPos * PK && kPfCols * 4 <= kPfPos * PK, "merge tables fit");
-  const int mc = tid >> 1, d0 = (tid & 1) * HD;
-  const int ti = mc / G, hg = mc % G;
-  const bool live = mc < BQ * G && ti < nq;
-  if (arrivals <= kPfMergeLds) {
-    if (tid < kPfCols) {
-      float mi[kPfMergeLds], li[kPfMergeLds];
+    if (t.lt > 0) {
+      bool ok[LPT];
+      if (tid == 0) s_bad = 0;
+      __syncthreads();   // the flag is cleared, and an earlier segment's last step is read
+      load_entries(j0);
+      load_rows(j0, ok);
+      load_entries(j0 + kPfPos < j1 ? j0 + kPfPos : j0);
+      store_rows(0, ok);
+      __syncthreads();
+    }
+    int buf = 0;
+    for (int jt = j0; jt < j1; jt += kPfPos, buf ^= 1) {
+      // the next step's rows and the table entries of the one after it, in flight across this
+      // step's products and softmax
+      const bool more = jt + kPfPos < j1;
+      bool ok[LPT];
+      if (more) {
+        load_rows(jt + kPfPos, ok);
+        load_entries(jt + 2 * kPfPos < j1 ? jt + 2 * kPfPos : jt);
+      }
+      if (live) {
+        const unsigned char* kt = s_k[buf] + c32 * PK + 16 * h;
+        const unsigned char* vt = s_v[buf] + tr_pos * PV + tr_dim * 2;
+        // S^T = K Q^T for the step's two 32-position row blocks (two independent MFMA chains)
+        f32x16_t st[2];
 #pragma unroll
-      for (int i = 0; i < kPfMergeLds; ++i) {
-        mi[i] = -INFINITY;
-        li[i] = 0.f;
-        if (i < arrivals) {
-          mi[i] = ld_dev(&f.ws_ml[((wbase + i) * kPfCols + tid) * 2]);
-          li[i] = ld_dev(&f.ws_ml[((wbase + i) * kPfCols + tid) * 2 + 1]);
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) st[rb][e] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+          for (int rb = 0; rb < 2; ++rb) {
+            const u32x4 x = *reinterpret_cast<const u32x4*>(kt + 32 * rb * PK + 32 * ks);
+            st[rb] = M::mma(__builtin_bit_cast(vec, x), qop[ks], st[rb]);
+          }
+        }
+        // the online softmax of the lane's column over the step's 64 positions (element e of block
+        // rb: position 32 rb + 8 (e / 4) + 4 h + e % 4; the other half in lane ^ 32)
+        const bool bad = s_bad != 0;
+        if (jt + kPfPos > kend_w || bad) {   // a position of the step hidden from a column
+#pragma unroll
+          for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              const int r = 32 * rb + 8 * (e >> 2) + 4 * h + (e & 3);
+              st[rb][e] = jt + r < kend ? st[rb][e] : -INFINITY;
+            }
+          if (bad) {   // look the step's blocks up again
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+              for (int e = 0; e < 16; ++e) {
+                const int j = jt + 32 * rb + 8 * (e >> 2) + 4 * h + (e & 3);
+                int o;
+                const int bi = split(j < j1 ? j : j1 - 1, o);
+                const int b = bi < p.max_blocks_per_seq ? bt_row[bi] : -1;
+                if (b < 0 || b >= p.num_blocks) st[rb][e] = -INFINITY;
+              }
+          }
+        }
+        float mt = -INFINITY;
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) mt = fmaxf(mt, st[rb][e]);
+        mt = fmaxf(mt, __shfl_xor(mt, 32)) * scale;
+        // The column's reference m moves only when a score exceeds it by more than 8 (log2 units),
+        // to the new maximum: weights stay at most 2^8 and the accumulators are rescaled rarely.
+        // exp2 by v_exp_f32 (a weight below 2^-126 flushes to zero); -inf scores weigh 0, and a
+        // column with no score yet subtracts 0.
+        const bool move = mt > m + 8.f;
+        const float mn = move ? mt : m;
+        const float msub = mn == -INFINITY ? 0.f : mn;
+        const float alpha = move ? __builtin_amdgcn_exp2f(m - msub) : 1.f;
+        m = mn;
+        if (__ballot(move) != 0ull) {   // a column's reference moved: rescale
+          l *= alpha;
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[db][e] *= alpha;
+        }
+        // per 16-position k-step s: P as the hi / lo B operands, then O^T += V^T P^T with the V^T
+        // operand of dim 32 db + c32 (k-slot i of half h at position 16 s + 8 (i / 4) + 4 h + i % 4)
+        // read from the value rows by two transposing reads (k-slots 0-3, then 4-7)
+        float ls = 0.f;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          u32x4 wh, wl;
+#pragma unroll
+          for (int i2 = 0; i2 < 4; ++i2) {
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(st[s >> 1][8 * (s & 1) + 2 * i2], scale, -msub));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(st[s >> 1][8 * (s & 1) + 2 * i2 + 1], scale, -msub));
+            ls += p0 + p1;
+            wh[i2] = M::pack2(p0, p1);
+            wl[i2] = M::pack2(p0 - M::lo(wh[i2]), p1 - M::hi(wh[i2]));
+          }
+          const vec phi = __builtin_bit_cast(vec, wh), plo = __builtin_bit_cast(vec, wl);
+#pragma unroll
+          for (int db = 0; db < DB; ++db) {
+            const unsigned char* src = vt + 16 * s * PV + 64 * db;
+            const u32x2 lo4 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                            (__attribute__((address_space(3))) i16x4*)(src)));
+            const u32x2 hi4 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                            (__attribute__((address_space(3))) i16x4*)(src + 8 * PV)));
+            const u32x4 x = {lo4[0], lo4[1], hi4[0], hi4[1]};
+            const vec a = __builtin_bit_cast(vec, x);
+            acc[db] = M::mma(a, phi, acc[db]);
+            acc[db] = M::mma(a, plo, acc[db]);
+          }
+        }
+        l += ls;   // this half's positions; the other half's sum is in lane ^ 32
+      }
+      if (more) store_rows(buf ^ 1, ok);
+      __syncthreads();   // the next step staged, this one read
+    }
+    l += __shfl_xor(l, 32);
+
+    // O^T layout: lane, element e -> column c, dim 32 db + 8 (e / 4) + 4 h + e % 4
+    const int64_t obase = (int64_t)(t.t0 + tok) * p.so_tok + (int64_t)(kvh * G + hd) * p.so_head + 4 * h;
+    auto write_out = [&](const f32x16_t (&o)[DB], float sum) {
+      if (kvl < 0) return;
+      const float inv = sum > 0.f ? 1.f / sum : 0.f;   // no visible key: zeros (the reference's l == 0 guard)
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+          float x[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] = sum > 0.f ? o[db][4 * e4 + i] * inv : 0.f;
+          const int64_t d = obase + 32 * db + 8 * e4;
+          if (f.out_vec) {
+            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.out) + d) =
+                u32x2{M::pack2(x[0], x[1]), M::pack2(x[2], x[3])};
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) store_one<T>(p.out, d + i, x[i]);
+          }
+        }
+    };
+    if (take == t.steps) {
+      write_out(acc, l);
+    } else {
+      // A cut tile: this segment's partials to its slot (agent-scope stores: the segments' workgroups
+      // run on different XCDs).  Workgroup i's slot for a tile begun by an earlier workgroup is i; for
+      // a tile it begins and does not finish, grid + (i or the (tile, KV head), whichever are fewer).
+      const int th = kvh * n_tiles + tile;
+      const int64_t us = u - off;   // the tile's first unit
+      const int wa = (int)(us / per), wb = (int)((us + t.steps - 1) / per);
+      const int begin_slot = f.grid + (f.grid <= n_tiles * p.hkv ? wa : th);
+      constexpr int SW = D / 2 * 64;   // floats of a slot per wave
+      const int mine = w == wa ? begin_slot : w;
+      if (live) {
+        float* dst = f.ws_acc + ((int64_t)mine * kPfWaves + wave) * SW + 2 * lane;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int e = 0; e < 16; e += 2) st_dev2(dst + (db * 16 + e) * 64, acc[db][e], acc[db][e + 1]);
+        if (h == 0) st_dev2(f.ws_ml + ((int64_t)mine * kPfCols + c) * 2, m, l);
+      }
+      // the last segment to arrive merges (the partials crossed through agent-scope atomic stores
+      // completed by the s_waitcnt, read back through agent-scope loads)
+      const int arrivals = wb - wa + 1;
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      int32_t* counter = f.counters + th;
+      if (tid == 0) s_last = atomicAdd(counter, 1) == arrivals - 1;
+      __syncthreads();
+      if (s_last) {
+        if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (live) {
+          float mx = -INFINITY;
+          for (int i = wa; i <= wb; ++i)
+            mx = fmaxf(mx, ld_dev2(f.ws_ml + ((int64_t)(i == wa ? begin_slot : i) * kPfCols + c) * 2)[0]);
+          float L = 0.f;
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
+          for (int i = wa; i <= wb; ++i) {
+            const int64_t slot = i == wa ? begin_slot : i;
+            const float* src = f.ws_acc + (slot * kPfWaves + wave) * SW + 2 * lane;
+            const f32x2 ml = ld_dev2(f.ws_ml + (slot * kPfCols + c) * 2);
+            f32x2 a[D / 4];   // all of a segment's loads issued before the first is used
+#pragma unroll
+            for (int e = 0; e < D / 4; ++e) a[e] = ld_dev2(src + e * 128);
+            // a segment whose keys were all skipped (m = -inf) weighs 0
+            const float wt = ml[0] == -INFINITY ? 0.f : exp2f(ml[0] - mx);
+            L = fmaf(wt, ml[1], L);
+#pragma unroll
+            for (int e = 0; e < D / 4; ++e) {
+              acc[e / 8][2 * (e % 8)] = fmaf(wt, a[e][0], acc[e / 8][2 * (e % 8)]);
+              acc[e / 8][2 * (e % 8) + 1] = fmaf(wt, a[e][1], acc[e / 8][2 * (e % 8) + 1]);
+            }
+          }
+          write_out(acc, L);
         }
       }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < kPfMergeLds; ++i) mx = fmaxf(mx, mi[i]);
-      float L = 0.f;
-#pragma unroll
-      for (int i = 0; i < kPfMergeLds; ++i) {
-        // a partition whose keys were all skipped (m = -inf) weighs 0
-        const float w = mi[i] == -INFINITY ? 0.f : exp2f(mi[i] - mx);
-        L = fmaf(w, li[i], L);
-        if (i < arrivals) s_w[i * kPfCols + tid] = w;
-      }
-      s_L[tid] = L;
     }
-    __syncthreads();
-    if (!live) return;
-    float o[HD];
-#pragma unroll
-    for (int d = 0; d < HD; ++d) o[d] = 0.f;
-    for (int i = 0; i < arrivals; ++i) {
-      const float w = s_w[i * kPfCols + mc];
-      const float* src = &f.ws_acc[((wbase + i) * kPfCols + mc) * D + d0];
-      float a[HD];
-#pragma unroll
-      for (int d = 0; d < HD; ++d) a[d] = ld_dev(src + d);
-#pragma unroll
-      for (int d = 0; d < HD; ++d) o[d] = fmaf(w, a[d], o[d]);
-    }
-    const float L = s_L[mc];
-    const int64_t ob = (int64_t)(t0 + ti) * p.so_tok + (int64_t)(kvh * G + hg) * p.so_head + d0;
-#pragma unroll
-    for (int d = 0; d < HD; ++d) store_one<T>(p.out, ob + d, L > 0.f ? o[d] / L : 0.f);
-    return;
+    u += take;
+    off = 0;
+    ++tile;
   }
-  // more partitions than the LDS table holds: one pass of max-rescaled sums per thread
-  if (!live) return;
-  float mm = -INFINITY, L = 0.f;
-  float o[HD];
-#pragma unroll
-  for (int d = 0; d < HD; ++d) o[d] = 0.f;
-  for (int i = 0; i < arrivals; ++i) {
-    const float mi = ld_dev(&f.ws_ml[((wbase + i) * kPfCols + mc) * 2]);
-    const float li = ld_dev(&f.ws_ml[((wbase + i) * kPfCols + mc) * 2 + 1]);
-    if (mi == -INFINITY) continue;
-    const float* src = &f.ws_acc[((wbase + i) * kPfCols + mc) * D + d0];
-    float a[HD];
-#pragma unroll
-    for (int d = 0; d < HD; ++d) a[d] = ld_dev(src + d);
-    if (mi > mm) {
-      const float r = mm == -INFINITY ? 0.f : exp2f(mm - mi);
-      L *= r;
-#pragma unroll
-      for (int d = 0; d < HD; ++d) o[d] *= r;
-      mm = mi;
-    }
-    const float w = exp2f(mi - mm);
-    L = fmaf(w, li, L);
-#pragma unroll
-    for (int d = 0; d < HD; ++d) o[d] = fmaf(w, a[d], o[d]);
-  }
-  const int64_t ob = (int64_t)(t0 + ti) * p.so_tok + (int64_t)(kvh * G + hg) * p.so_head + d0;
-#pragma unroll
-  for (int d = 0; d < HD; ++d) store_one<T>(p.out, ob + d, L > 0.f ? o[d] / L : 0.f);
 }
 
 // ---- host side ---------------------------------------------------------------------------------
@@ -936,13 +1045,28 @@ int pf_part_tokens_for(int32_t n_tiles, int32_t hkv, int32_t max_seq_len) {
   return part;
 }
 
-// Bytes of the prefill tiles' partials (0 when every tile fits one partition).
-uint64_t pf_workspace_bytes(int32_t n_tiles, int32_t hkv, int32_t head_dim, int32_t max_seq_len) {
+// Workgroups that share the steps of the prefill tiles, or 0 for one workgroup per (tile, KV head):
+// tiles are cut when the longest could be (max_seq_len above the partition length above, which
+// shrinks while there are fewer than 512 of them).  512 workgroups are all resident at once, so
+// equal shares end together.  Fewer, so that the slots they need stay within the partials' room
+// of one slot per (tile, KV head, partition).
+int pf_grid_for(int32_t n_tiles, int32_t hkv, int32_t max_seq_len) {
   if (n_tiles <= 0) return 0;
   const int part = pf_part_tokens_for(n_tiles, hkv, max_seq_len);
-  const int64_t max_parts = ((int64_t)max_seq_len + part - 1) / part;
-  if (max_parts <= 1) return 0;
-  return (uint64_t)n_tiles * hkv * max_parts * kPfCols * (head_dim + 2) * sizeof(float);
+  const int64_t parts = ((int64_t)max_seq_len + part - 1) / part;
+  if (parts <= 1) return 0;
+  const int64_t th = (int64_t)n_tiles * hkv;
+  return (int)(th * (parts - 1) < kPfTargetGroups ? th * (parts - 1) : kPfTargetGroups);
+}
+
+// Bytes of the prefill tiles' partials (0 when no tile is cut): a slot per workgroup for a tile
+// begun by another, and one per workgroup or (tile, KV head), whichever are fewer, for a tile begun
+// and not finished.
+uint64_t pf_workspace_bytes(int32_t n_tiles, int32_t hkv, int32_t head_dim, int32_t max_seq_len) {
+  const int64_t grid = pf_grid_for(n_tiles, hkv, max_seq_len);
+  if (grid == 0) return 0;
+  const int64_t th = (int64_t)n_tiles * hkv;
+  return (uint64_t)(grid + (grid < th ? grid : th)) * kPfCols * (head_dim + 2) * sizeof(float);
 }
 
 int part_tokens_for(int32_t total_q, int32_t hkv, int32_t max_seq_len) {
@@ -991,7 +1115,7 @@ void launch(const PaParams& p, const PfParams& f, int n_tokens, int n_tiles, hip
   }
   if constexpr (Elem<T>::bytes == 2) {
     if (n_tiles > 0) {
-      dim3 grid(n_tiles, p.hkv, f.max_parts);
+      const dim3 grid((unsigned)(f.grid > 0 ? f.grid : n_tiles * p.hkv));
       hipLaunchKernelGGL((pa_prefill_kernel<T, D, G>), grid, dim3(kPfThreads), 0, stream, p, f);
     }
   }
@@ -1135,11 +1259,17 @@ int ns_paged_attention(const ns_paged_attn_args* a, hipStream_t stream) {
   PfParams f;
   f.tiles = a->prefill_tiles;
   char* ws = reinterpret_cast<char*>(a->workspace);
+  f.grid = pf_grid_for(n_tiles, a->num_kv_heads, a->max_seq_len);
+  if (((uintptr_t)a->workspace + need) % 8 != 0) f.grid = 0;   // the partials go in 8-byte pieces
+  f.n_tiles = n_tiles;
   f.ws_acc = pf_need ? reinterpret_cast<float*>(ws + need) : nullptr;
-  f.ws_ml = pf_need ? f.ws_acc + (uint64_t)n_tiles * a->num_kv_heads * pf_max_parts * kPfCols * a->head_dim : nullptr;
+  f.ws_ml = pf_need ? f.ws_acc + pf_need / sizeof(float) / (a->head_dim + 2) * a->head_dim : nullptr;
   f.counters = a->counters ? a->counters + (int64_t)a->total_q * a->num_kv_heads : nullptr;
-  f.part_tokens = pf_part;
-  f.max_parts = pf_max_parts > 0 ? (int32_t)pf_max_parts : 1;
+  f.cap = (pf_max_parts > 0 ? pf_max_parts : 1) * pf_part;
+  f.scale_log2 = a->scale == 0.f ? 1.f : fabsf(a->scale) * kLog2e;
+  f.q_and = a->scale == 0.f ? 0u : 0xffffffffu;
+  f.q_xor = a->scale < 0.f ? 0x80008000u : 0u;
+  f.out_vec = (uintptr_t)a->out % 8 == 0 && a->stride_o_token % 4 == 0 && a->stride_o_head % 4 == 0;
 
   const int g = a->num_heads_q / a->num_kv_heads;
   switch (a->dtype) {

@@ -276,3 +276,32 @@ def test_prefill_tile_merged_from_many_partitions(device, d):
     # holds (the one-pass rescaled merge) and a 4000-position tile into fewer (the table)
     case = make_case(97 + d, [9000, 4000], [20, 30], d=d)
     check(case, device)
+
+
+@pytest.mark.parametrize("seqs,qlens,scale,bad", [
+    ([3000, 65, 70, 64, 63], [500, 65, 2, 64, 3], 1.0, False),        # tiles cut mid-way, others whole beside them
+    ([20000], [2], 1.0, False),                                       # a tile shared by many workgroups
+    ([40, 1, 33, 2] * 70, [20, 1, 33, 2] * 70, 1.0, False),           # more tiles than threads, shares of several tiles
+    ([1300, 257], [130, 257], -0.5, False),                           # a negative score scale
+    ([1300, 257], [130, 257], 0.0, False),                            # and none
+    ([1300, 500], [130, 200], 1.0, True),                             # blocks outside the cache in a cut tile
+])
+def test_prefill_shared_steps(device, seqs, qlens, scale, bad):
+    # the steps of all tiles are shared evenly by the workgroups, whatever the tiles' lengths
+    case = make_case(len(seqs) + seqs[0], seqs, qlens)
+    case["scale"] *= scale
+    if bad:
+        case["block_tables"][0, 3:9:2] = 10 ** 6
+        case["block_tables"][1, 20] = -3
+    # an output whose rows are not 8-byte aligned, next to the plain one
+    c = to_device(case, device)
+    q = c["query"]
+    wide = torch.empty((q.shape[0], q.shape[1], q.shape[2] + 1), dtype=q.dtype, device=device)
+    a = run(case, device)
+    b = run(case, device, out=wide[:, :, 1:])
+    assert torch.equal(a, b)
+    if bad:   # the per-token kernel skips the same keys
+        ref = run(case, device, max_query_len=1).double()
+        assert ((a.double() - ref).abs() <= 1e-4 + 2.0 ** -7 * ref.abs()).all()
+    else:
+        assert_close_to_oracle(a, PA.paged_attention(**oracle_args(case), terms=True), q.dtype)
