@@ -514,7 +514,8 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
 // the sequences' lengths and a tile is cut only where a run ends: at most two partials per
 // workgroup, stored and merged in the lanes' accumulator layout (256 contiguous bytes per 4-byte
 // element of a wave).  Four 512-token chunks ending at 2048 .. 8192 positions (24 / 8 heads of 128
-// dims, bf16): 627 -> 257 us, 195 -> 475 TFLOP/s, against partitions of at most 1024 positions whose
+// dims, bf16): 627 -> 257 us, 195 -> 475 TFLOP/s (223 us, 545 TFLOP/s with scalar row addresses),
+// against partitions of at most 1024 positions whose
 // 64 KB of partials each went out and came back as scattered 4-byte accesses; three chunks of up to
 // 417 tokens beside 29 decode rows (32 / 8 heads of 64 dims, f16): 89 -> 55 us for the call.
 // Keys and values are double buffered in LDS (one barrier a step), the value rows at a pitch under
@@ -622,7 +623,11 @@ __device__ __forceinline__ f32x2 ld_dev2(const float* p) {
   return f32x2{__uint_as_float((uint32_t)w), __uint_as_float((uint32_t)(w >> 32))};
 }
 
-template <typename T, int D, int G>
+// BW: the block size is a power of two and at least the consecutive positions one load instruction
+// of a wave covers (4 at 128 dims, 8 at 64), so these never straddle two blocks: the block is the
+// wave's, and a row's address a scalar address plus a lane's fixed offset instead of 64-bit products
+// per lane (four 512-token chunks up to 8192 positions: 252 -> 223 us).
+template <typename T, int D, int G, bool BW>
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void pa_prefill_kernel(PaParams p,
                                                                                                         PfParams f) {
   using M = Mma<T>;
@@ -681,7 +686,8 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     const int64_t U = S * p.hkv;
     per = (U + f.grid - 1) / f.grid;
     if (per < kPfMinSteps) per = kPfMinSteps;
-    w = blockIdx.x;
+    // consecutive runs on one XCD: they read the same KV head's rows
+    w = f.grid % 8 == 0 ? (int)(blockIdx.x % 8) * (f.grid / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
     u0 = per * w;
     u1 = u0 + per < U ? u0 + per : U;
     if (u0 >= U) return;
@@ -717,6 +723,10 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
   // keeps token strides times block_size below 2^31, so a slot's offset is a 32-bit product
   const int dc0 = tid % CPP;
   const int sk_tok = (int)p.sk_tok, sv_tok = (int)p.sv_tok;
+  constexpr int PW = 64 / CPP;   // positions of a wave's load instruction
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const uint32_t koff = (uint32_t)(lane / CPP * sk_tok) * 2u + 16u * dc0;
+  const uint32_t voff = (uint32_t)(lane / CPP * sv_tok) * 2u + 16u * dc0;
   // The transposing read (ds_read_b64_tr_b16): in each 16-lane group, lane j's four results are
   // element j % 4 of the 4-element rows that lanes 4 m + j / 4 address, m = 0..3.  So that lane L
   // receives positions 16 s + 4 h + m of dim 32 db + L % 32, lane L addresses position
@@ -755,8 +765,8 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
     for (int sh = 1; sh < 64; sh <<= 1) kend_w = min(kend_w, __shfl_xor(kend_w, sh));
     const int32_t* bt_row = p.bt + (int64_t)t.seq * p.sbt;
-    const char* kbase = reinterpret_cast<const char*>(p.k) + ((int64_t)kvh * p.sk_head + 8 * dc0) * 2;
-    const char* vbase = reinterpret_cast<const char*>(p.v) + ((int64_t)kvh * p.sv_head + 8 * dc0) * 2;
+    const char* kbase = reinterpret_cast<const char*>(p.k) + (int64_t)kvh * p.sk_head * 2;
+    const char* vbase = reinterpret_cast<const char*>(p.v) + (int64_t)kvh * p.sv_head * 2;
 
     // Q^T operand: column c, dims 16 ks + 8 h .. + 7 (zeros for a padding column)
     vec qop[KS];
@@ -777,46 +787,61 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     // position (tid + kPfThreads r) / CPP of a step.
     auto split = [&](int j, int& o) -> int {
       int bi;
-      if (p.bs_shift >= 0) { bi = j >> p.bs_shift; o = j & (p.block_size - 1); }
+      if (BW || p.bs_shift >= 0) { bi = j >> p.bs_shift; o = j & (p.block_size - 1); }
       else { bi = j / p.block_size; o = j - bi * p.block_size; }
       return bi;
     };
-    auto entry = [&](int jt, int r) -> int {   // -1: past the segment or the table
-      const int j = jt + (tid + kPfThreads * r) / CPP;
-      int o;
-      const int bi = split(j < j1 ? j : j1 - 1, o);
-      return j < j1 && bi < p.max_blocks_per_seq ? bt_row[bi] : -1;
-    };
     u32x4 kreg[LPT], vreg[LPT];
     int blk[LPT];
-    auto load_entries = [&](int jt) {
-#pragma unroll
-      for (int r = 0; r < LPT; ++r) blk[r] = entry(jt, r);
-    };
-    auto load_rows = [&](int jt, bool (&ok)[LPT]) {
+    uint32_t bad_rows = 0u;   // bit r: chunk r's block is invalid
+    // the first position of the wave's group for chunk r of the step at jt; past the segment, its last group
+    auto group_of = [&](int jt, int r) -> int { return min(jt + wv * PW + kPfThreads / CPP * r, (j1 - 1) & -PW); };
+    auto load_entries = [&](int jt) {   // -1: past the table
 #pragma unroll
       for (int r = 0; r < LPT; ++r) {
-        const int j = jt + (tid + kPfThreads * r) / CPP;
         int o;
-        split(j < j1 ? j : j1 - 1, o);
-        ok[r] = blk[r] >= 0 && blk[r] < p.num_blocks;
-        if (j < j1 && !ok[r]) {
-          s_bad = 1;
-          if (p.status) atomicOr(p.status, NS_PA_STATUS_BAD_BLOCK);
-        }
-        const int b = ok[r] ? blk[r] : 0;   // block 0 stands in for an invalid one; its rows are not used
-        kreg[r] = *reinterpret_cast<const u32x4*>(kbase + ((int64_t)b * p.sk_blk + o * sk_tok) * 2);
-        vreg[r] = *reinterpret_cast<const u32x4*>(vbase + ((int64_t)b * p.sv_blk + o * sv_tok) * 2);
+        const int bi = split(BW ? group_of(jt, r) : min(jt + (tid + kPfThreads * r) / CPP, j1 - 1), o);
+        blk[r] = bi < p.max_blocks_per_seq ? bt_row[bi] : -1;
       }
     };
-    auto store_rows = [&](int buf, const bool (&ok)[LPT]) {
+    auto load_rows = [&](int jt) {
+      bad_rows = 0u;
+#pragma unroll
+      for (int r = 0; r < LPT; ++r) {
+        int o;
+        split(BW ? group_of(jt, r) : min(jt + (tid + kPfThreads * r) / CPP, j1 - 1), o);
+        int b = BW ? __builtin_amdgcn_readfirstlane(blk[r]) : blk[r];
+        // an invalid entry of the segment (past its end, its last one again): block 0 stands in, the
+        // rows are not used
+        const bool bad = (uint32_t)b >= (uint32_t)p.num_blocks;
+        b = bad ? 0 : b;
+        bad_rows |= bad ? 1u << r : 0u;
+        if constexpr (BW) {   // block strides below 2^31: one 32 x 32 bit product each
+          kreg[r] = *reinterpret_cast<const u32x4*>(
+              kbase + ((uint64_t)(uint32_t)b * (uint32_t)p.sk_blk + (uint32_t)(o * sk_tok)) * 2 + koff);
+          vreg[r] = *reinterpret_cast<const u32x4*>(
+              vbase + ((uint64_t)(uint32_t)b * (uint32_t)p.sv_blk + (uint32_t)(o * sv_tok)) * 2 + voff);
+        } else {
+          kreg[r] = *reinterpret_cast<const u32x4*>(kbase + ((int64_t)b * p.sk_blk + o * sk_tok) * 2 + 16 * dc0);
+          vreg[r] = *reinterpret_cast<const u32x4*>(vbase + ((int64_t)b * p.sv_blk + o * sv_tok) * 2 + 16 * dc0);
+        }
+      }
+      if (bad_rows != 0u) {
+        s_bad = 1;
+        if (p.status) atomicOr(p.status, NS_PA_STATUS_BAD_BLOCK);
+      }
+    };
+    auto store_rows = [&](int jt, int buf) {
+      if (bad_rows != 0u || jt + kPfPos > j1) {   // weight 0 times a row not of this sequence must be 0
+#pragma unroll
+        for (int r = 0; r < LPT; ++r)
+          if (((bad_rows >> r) & 1u) || jt + (tid + kPfThreads * r) / CPP >= j1) vreg[r] = u32x4{0u, 0u, 0u, 0u};
+      }
 #pragma unroll
       for (int r = 0; r < LPT; ++r) {
         const int pos = (tid + kPfThreads * r) / CPP;
-        u32x4 x = vreg[r];
-        if (!ok[r]) x = u32x4{0u, 0u, 0u, 0u};   // weight 0 times a row not of this sequence must be 0
         *reinterpret_cast<u32x4*>(s_k[buf] + pos * PK + dc0 * 16) = kreg[r];
-        *reinterpret_cast<u32x4*>(s_v[buf] + pos * PV + dc0 * 16) = x;
+        *reinterpret_cast<u32x4*>(s_v[buf] + pos * PV + dc0 * 16) = vreg[r];
       }
     };
 
@@ -828,13 +853,12 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     float m = -INFINITY, l = 0.f;
 
     if (t.lt > 0) {
-      bool ok[LPT];
       if (tid == 0) s_bad = 0;
       __syncthreads();   // the flag is cleared, and an earlier segment's last step is read
       load_entries(j0);
-      load_rows(j0, ok);
-      load_entries(j0 + kPfPos < j1 ? j0 + kPfPos : j0);
-      store_rows(0, ok);
+      load_rows(j0);
+      load_entries(j0 + kPfPos);
+      store_rows(j0, 0);
       __syncthreads();
     }
     int buf = 0;
@@ -842,10 +866,9 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
       // the next step's rows and the table entries of the one after it, in flight across this
       // step's products and softmax
       const bool more = jt + kPfPos < j1;
-      bool ok[LPT];
       if (more) {
-        load_rows(jt + kPfPos, ok);
-        load_entries(jt + 2 * kPfPos < j1 ? jt + 2 * kPfPos : jt);
+        load_rows(jt + kPfPos);
+        load_entries(jt + 2 * kPfPos);
       }
       if (live) {
         const unsigned char* kt = s_k[buf] + c32 * PK + 16 * h;
@@ -941,7 +964,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
         }
         l += ls;   // this half's positions; the other half's sum is in lane ^ 32
       }
-      if (more) store_rows(buf ^ 1, ok);
+      if (more) store_rows(jt + kPfPos, buf ^ 1);
       __syncthreads();   // the next step staged, this one read
     }
     l += __shfl_xor(l, 32);
@@ -1116,7 +1139,11 @@ void launch(const PaParams& p, const PfParams& f, int n_tokens, int n_tiles, hip
   if constexpr (Elem<T>::bytes == 2) {
     if (n_tiles > 0) {
       const dim3 grid((unsigned)(f.grid > 0 ? f.grid : n_tiles * p.hkv));
-      hipLaunchKernelGGL((pa_prefill_kernel<T, D, G>), grid, dim3(kPfThreads), 0, stream, p, f);
+      if (p.bs_shift >= 0 && p.block_size >= 512 / D && p.sk_blk >= 0 && p.sv_blk >= 0 && p.sk_blk < INT32_MAX &&
+          p.sv_blk < INT32_MAX)
+        hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, true>), grid, dim3(kPfThreads), 0, stream, p, f);
+      else
+        hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, false>), grid, dim3(kPfThreads), 0, stream, p, f);
     }
   }
 }

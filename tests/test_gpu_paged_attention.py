@@ -202,6 +202,14 @@ def test_prefill_tiles_block_sizes(device, block_size):
     check(case, device)
 
 
+@pytest.mark.parametrize("d,block_size", [(128, 2), (128, 4), (128, 12), (128, 128), (64, 4), (64, 8), (64, 24)])
+def test_prefill_row_addresses_by_block_size(device, d, block_size):
+    # block sizes on both sides of the rule for scalar row addresses (a power of two of at least
+    # 512 / d positions), lengths that end inside a block
+    case = make_case(71 + block_size + d, [701, 77], [64, 77], d=d, block_size=block_size)
+    check(case, device)
+
+
 def test_prefill_tiles_repeat_bit_exact_and_strided_query(device):
     case = make_case(80, [900, 64], [300, 64], qkv_view=True)
     a = check(case, device)
