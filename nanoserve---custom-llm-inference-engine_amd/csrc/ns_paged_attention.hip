@@ -8,7 +8,8 @@
 //  * One 256-thread workgroup per (query token, KV head, KV partition) computes every query head of
 //    that KV head (G = num_heads_q / num_kv_heads of them), so each key and value row is read from
 //    HBM once per query token instead of once per query head as the reference's per-(token, head)
-//    programs do. Decode attention moves ~4 flops per byte: HBM bound, VALU arithmetic.
+//    programs do.  The 16-bit types take pa_decode_kernel (matrix core), float32 pa_partition_kernel
+//    (vector arithmetic; the two points below are its).
 //  * Lane layout per wave step: 16 KV positions, 8 lanes per position, each lane holding a
 //    head_dim/8 slice (32 contiguous bytes of a bf16 row at head_dim 128: two 16-byte loads). The
 //    slice's partial dot products are summed across the 8 lanes with ds_swizzle (no LDS traffic).
@@ -198,11 +199,19 @@ struct QueryPlace {
 // their start with the next one, so the largest index is the one that owns qi), as the reference's
 // repeat_interleave over query_lens (paged_attention_triton.py:109-112); its KV position
 // seq_len - q_len + (qi - start) (:115-131), the causal and in-sequence cuts (:64-66).
+// Searched by the whole wave, 64 entries at a time: one load for up to 64 sequences, two for up to
+// 4096, where a binary search is a chain of log2 of them.
 __device__ __forceinline__ QueryPlace place_query(const PaParams& p, int qi) {
-  int lo = 0, hi = p.num_seqs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (p.qsl[mid] <= qi) lo = mid; else hi = mid - 1;
+  const int lane = threadIdx.x & 63;
+  int lo = 0, len = p.num_seqs;
+  for (;;) {
+    const int stride = (len + 63) / 64;
+    const int at = lane * stride;
+    const int below = __popcll(__ballot(at < len && p.qsl[lo + (at < len ? at : 0)] <= qi));
+    const int skip = (below > 0 ? below - 1 : 0) * stride;
+    lo += skip;
+    if (stride == 1) break;
+    len = min(stride, len - skip);
   }
   const int seq_len = p.seq_lens[lo];
   const int kv_pos = seq_len - p.qlens[lo] + (qi - p.qsl[lo]);
@@ -211,7 +220,161 @@ __device__ __forceinline__ QueryPlace place_query(const PaParams& p, int qi) {
   return {lo, kv_len};
 }
 
+// ---- matrix core ------------------------------------------------------------------------------
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+
+// The MFMA and the 16-bit type's conversions: pack2 rounds two floats to nearest even into one
+// word (low half the first; v_cvt_pk_bf16_f32 for bfloat16), lo / hi widen a word's halves back.
+template <typename T> struct Mma;
+template <> struct Mma<Bf16> {
+  typedef bf16x8_t vec;
+  static __device__ __forceinline__ f32x4_t mma16(vec a, vec b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4_t mma16(u32x2 a, u32x2 b, f32x4_t c) {   // k = 16
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, a), __builtin_bit_cast(i16x4, b), c, 0,
+                                                     0, 0);
+  }
+  static __device__ __forceinline__ f32x16_t mma(vec a, vec b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2_t));
+  }
+  static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
+  static __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+};
+template <> struct Mma<F16> {
+  typedef f16x8_t vec;
+  static __device__ __forceinline__ f32x4_t mma16(vec a, vec b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4_t mma16(u32x2 a, u32x2 b, f32x4_t c) {   // k = 16
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4_t, a), __builtin_bit_cast(f16x4_t, b), c, 0, 0,
+                                                 0);
+  }
+  static __device__ __forceinline__ f32x16_t mma(vec a, vec b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2_t));
+  }
+  static __device__ __forceinline__ float lo(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)w); }
+  static __device__ __forceinline__ float hi(uint32_t w) {
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+  }
+};
+
 // ---- partition kernel ---------------------------------------------------------------------------
+
+// The end of a partition: the sum over the waves of red(wave, head, dim), s_m and s_l the partition's
+// maximum (log2 units) and sum of weights per head.  s_w: G * kMaxMerge floats of LDS, free once red
+// has been read.
+template <typename T, int D, int G, int kMaxMerge, typename Red>
+__device__ __forceinline__ void finish_partition(const PaParams& p, int qi, int kvh, int part, int n_parts, Red red,
+                                                 float* s_m, float* s_l, float* s_w) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const bool direct = n_parts == 1;
+  for (int e = threadIdx.x; e < G * D; e += kThreads) {
+    const int g = e / D, d = e % D;
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) o += red(w, g, d);
+    const int h = kvh * G + g;
+    if (direct) {
+      const float l = s_l[g];
+      store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
+    } else if (p.ws_acc && part < p.max_parts) {
+      const int64_t slot_idx = ((int64_t)qi * p.hq + h) * p.max_parts + part;
+      st_dev(&p.ws_acc[slot_idx * D + d], o);
+      if (d == 0) {
+        st_dev(&p.ws_ml[slot_idx * 2], s_m[g]);
+        st_dev(&p.ws_ml[slot_idx * 2 + 1], s_l[g]);
+      }
+    }
+  }
+  if (direct || !p.ws_acc || part >= p.max_parts) return;
+
+  // Split row: the last of its partitions to arrive merges them (max-rescaled sums, one pass)
+  // and resets the row's counter. Every store above completes before the counter moves.
+  const int arrivals = n_parts < p.max_parts ? n_parts : p.max_parts;
+  __shared__ int s_last;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  int32_t* counter = p.counters + (int64_t)qi * p.hkv + kvh;
+  // The partials went out through agent-scope atomic stores (served at the device coherence
+  // point, past the per-XCD L2s) completed by the s_waitcnt above, and are read back through
+  // agent-scope atomic loads, so the ticket needs no release / acquire fence (a buffer_wbl2 /
+  // buffer_inv of the whole L2: 106 -> 128 us at 64 x 2048 decode).
+  if (threadIdx.x == 0) s_last = atomicAdd(counter, 1) == arrivals - 1;
+  __syncthreads();
+  if (!s_last) return;
+  if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (arrivals <= kMaxMerge) {
+    // weights w_i / L of the partitions into LDS (one wave per head, lanes over partitions), then
+    // every output is an independent weighted sum of the partitions' unnormalised outputs
+    for (int g = wave; g < G; g += kWaves) {
+      const int64_t base = ((int64_t)qi * p.hq + kvh * G + g) * p.max_parts;
+      float m = -INFINITY;
+      for (int i = lane; i < arrivals; i += 64) m = fmaxf(m, ld_dev(&p.ws_ml[(base + i) * 2]));
+      m = wave_max(m);
+      float l = 0.f;
+      for (int i = lane; i < arrivals; i += 64) {
+        const float mi = ld_dev(&p.ws_ml[(base + i) * 2]);
+        const float w = (m == -INFINITY || mi == -INFINITY) ? 0.f : exp2f(mi - m);
+        s_w[g * kMaxMerge + i] = w;
+        l = fmaf(w, ld_dev(&p.ws_ml[(base + i) * 2 + 1]), l);
+      }
+      l = wave_sum(l);
+      if (lane == 0) s_l[g] = l;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < G * D; e += kThreads) {
+      const int g = e / D, d = e % D;
+      const int h = kvh * G + g;
+      const int64_t base = ((int64_t)qi * p.hq + h) * p.max_parts;
+      float o = 0.f;
+#pragma unroll 4
+      for (int i = 0; i < arrivals; ++i) o = fmaf(s_w[g * kMaxMerge + i], ld_dev(&p.ws_acc[(base + i) * D + d]), o);
+      const float l = s_l[g];
+      store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
+    }
+    return;
+  }
+  // more partitions than the LDS weight table holds: one pass of max-rescaled sums per output
+  for (int e = threadIdx.x; e < G * D; e += kThreads) {
+    const int g = e / D, d = e % D;
+    const int h = kvh * G + g;
+    const int64_t base = ((int64_t)qi * p.hq + h) * p.max_parts;
+    float m = -INFINITY, l = 0.f, o = 0.f;
+    for (int i = 0; i < arrivals; ++i) {
+      const float mi = ld_dev(&p.ws_ml[(base + i) * 2]);
+      const float li = ld_dev(&p.ws_ml[(base + i) * 2 + 1]);
+      const float ai = ld_dev(&p.ws_acc[(base + i) * D + d]);
+      if (mi == -INFINITY) continue;  // a partition whose keys were all skipped
+      if (mi > m) {
+        const float r = m == -INFINITY ? 0.f : exp2f(m - mi);
+        l *= r;
+        o *= r;
+        m = mi;
+      }
+      const float w = exp2f(mi - m);
+      l = fmaf(w, li, l);
+      o = fmaf(w, ai, o);
+    }
+    store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
+  }
+}
 
 template <typename T, int D, int G>
 __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
@@ -393,96 +556,299 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   }
   __syncthreads();
 
-  const bool direct = n_parts == 1;
-  for (int e = threadIdx.x; e < G * D; e += kThreads) {
-    const int g = e / D, d = e % D;
-    float o = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) o += s_red[(w * G + g) * D + d];
-    const int h = kvh * G + g;
-    if (direct) {
-      const float l = s_l[g];
-      store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
-    } else if (p.ws_acc && part < p.max_parts) {
-      const int64_t slot_idx = ((int64_t)qi * p.hq + h) * p.max_parts + part;
-      st_dev(&p.ws_acc[slot_idx * D + d], o);
-      if (d == 0) {
-        st_dev(&p.ws_ml[slot_idx * 2], s_m[g]);
-        st_dev(&p.ws_ml[slot_idx * 2 + 1], s_l[g]);
-      }
-    }
-  }
-  if (direct || !p.ws_acc || part >= p.max_parts) return;
+  finish_partition<T, D, G, kMaxPart>(p, qi, kvh, part, n_parts,
+                                      [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_score);
+}
 
-  // Split row: the last of its partitions to arrive merges them (max-rescaled sums, one pass)
-  // and resets the row's counter. Every store above completes before the counter moves.
-  const int arrivals = n_parts < p.max_parts ? n_parts : p.max_parts;
-  __shared__ int s_last;
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  int32_t* counter = p.counters + (int64_t)qi * p.hkv + kvh;
-  // The partials went out through agent-scope atomic stores (served at the device coherence
-  // point, past the per-XCD L2s) completed by the s_waitcnt above, and are read back through
-  // agent-scope atomic loads, so the ticket needs no release / acquire fence (a buffer_wbl2 /
-  // buffer_inv of the whole L2: 106 -> 128 us at 64 x 2048 decode).
-  if (threadIdx.x == 0) s_last = atomicAdd(counter, 1) == arrivals - 1;
-  __syncthreads();
-  if (!s_last) return;
-  if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (arrivals <= kMaxPart) {
-    // weights w_i / L of the partitions into LDS (one wave per head, lanes over partitions), then
-    // every output is an independent weighted sum of the partitions' unnormalised outputs
-    for (int g = wave; g < G; g += kWaves) {
-      const int64_t base = ((int64_t)qi * p.hq + kvh * G + g) * p.max_parts;
-      float m = -INFINITY;
-      for (int i = lane; i < arrivals; i += 64) m = fmaxf(m, ld_dev(&p.ws_ml[(base + i) * 2]));
-      m = wave_max(m);
-      float l = 0.f;
-      for (int i = lane; i < arrivals; i += 64) {
-        const float mi = ld_dev(&p.ws_ml[(base + i) * 2]);
-        const float w = (m == -INFINITY || mi == -INFINITY) ? 0.f : exp2f(mi - m);
-        s_score[g * kMaxPart + i] = w;
-        l = fmaf(w, ld_dev(&p.ws_ml[(base + i) * 2 + 1]), l);
-      }
-      l = wave_sum(l);
-      if (lane == 0) s_l[g] = l;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < G * D; e += kThreads) {
-      const int g = e / D, d = e % D;
-      const int h = kvh * G + g;
-      const int64_t base = ((int64_t)qi * p.hq + h) * p.max_parts;
-      float o = 0.f;
-#pragma unroll 4
-      for (int i = 0; i < arrivals; ++i) o = fmaf(s_score[g * kMaxPart + i], ld_dev(&p.ws_acc[(base + i) * D + d]), o);
-      const float l = s_l[g];
-      store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
+// The 16-bit types' partition kernel: the same workgroups, partitions, partials and merge, with the
+// products on the matrix core (v_mfma_f32_16x16x32, columns the G query heads padded to 16) and the
+// softmax online per wave, so that the waves stream independently and meet once at the end.  The
+// vector unit did about 165 instructions per 8 positions at G = 3 (the dot products, their lane sums,
+// the widening) and the passes of all the workgroups of a launch fell together, so that the memory
+// pipe idled across the softmax.
+//   * A wave takes steps of 32 positions.  A load instruction of
+//     a wave covers whole rows (4 of 128 dims, 8 of 64), so that every 128-byte line is taken at one
+//     touch: loading the products' operand layout (16 rows by 64 bytes) directly, with 128 KB in flight
+//     on a CU, evicted lines between their touches (64 x 2048 at G = 3: 114 us, and 105 at half the
+//     waves).  A step's loads are issued before the previous step's arithmetic (8 KB a wave in flight)
+//     and go through the wave's own LDS rows.
+//   * S^T: lane l holds head l % 16 at positions 16 b + 4 (l / 16) + i of row block b.  Its weights are
+//     the B operand of O^T += V^T P^T as they are, with k-slot i of quarter l / 16 at position
+//     4 (l / 16) + i for i < 4, else 12 + 4 (l / 16) + i; the V^T operand is read in that order by two
+//     transposing reads from the wave's own LDS rows.  P goes in as a high and a low 16-bit part, as in
+//     the prefill kernel.
+//   * LDS rows are unpadded; 16-byte chunk c of row r sits at c ^ swz(r), under which the 16 rows of a
+//     write and the 8 rows of a transposing read hit the 64 banks once.
+// Bound by HBM.  Measured (bf16, 8 KV heads of 128 dims, blocks of 16; the vector form, then this):
+// 8 x 8192 at G = 3: 61 -> 58 us; 64 x 2048: 107 -> 107 (5.0 TB/s); 256 rows of up to 512: 77 -> 57;
+// G = 4, 64 rows of up to 2048: 130 -> 80; G = 8, 32 rows of up to 2048: 134 -> 37.  At 128 dims three
+// waves a SIMD (168 registers): four spill 8 bytes and measured 63, 111 and 63 us on the first three,
+// two 61, 103 and 60.
+// BW as in the prefill kernel: a row's address is a scalar plus a lane's fixed offset.
+template <typename T, int D, int G, bool BW>
+__global__ __launch_bounds__(kThreads)
+    __attribute__((amdgpu_waves_per_eu(D == 128 ? 3 : 4, D == 128 ? 3 : 4))) void pa_decode_kernel(PaParams p) {
+  using M = Mma<T>;
+  using vec = typename M::vec;
+  constexpr int KS = D / 32;            // k-steps of S^T, and 16-byte chunks of a row per lane
+  constexpr int DB = D / 16;            // 16-dim blocks of O^T
+  constexpr int NB = D == 128 ? 1 : 2;  // 16-row blocks of a wave's step
+  constexpr int kStep = 16 * NB;        // its positions
+  constexpr uint32_t kAllOk = NB == 1 ? 0xffffu : 0xffffffffu;
+  constexpr int kMaxMerge = kMaxPart / 4;
+  static_assert(G <= 16, "the heads are the 16 columns");
+  __shared__ __align__(16) unsigned char s_kv[kWaves][2][kStep * D * 2];   // then the waves' outputs, then merge weights
+  __shared__ float s_wm[kWaves][G], s_wl[kWaves][G];
+  __shared__ float s_m[G], s_l[G];
+  __shared__ int s_blk[kMaxPart + 2];   // physical block of each block-table entry the partition spans
+  static_assert(sizeof(s_kv) >= (size_t)kWaves * G * D * 4 && sizeof(s_kv) >= (size_t)G * kMaxMerge * 4, "reuse");
+
+  const int qi = p.tokens != nullptr ? p.tokens[blockIdx.x] : (int)blockIdx.x;
+  const int kvh = blockIdx.y, part = blockIdx.z;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (qi < 0 || qi >= p.total_q) {   // a listed token outside the batch: flagged, nothing touched
+    if (threadIdx.x == 0 && part == 0 && kvh == 0 && p.status) atomicOr(p.status, NS_PA_STATUS_BAD_TILE);
+    return;
+  }
+  const QueryPlace qp = place_query(p, qi);
+  const int n_parts = (qp.kv_len + p.part_tokens - 1) / p.part_tokens;
+  if (part == 0 && n_parts > p.max_parts && threadIdx.x == 0 && p.status)
+    atomicOr(p.status, NS_PA_STATUS_SEQ_TOO_LONG);
+  if (part >= n_parts) {
+    if (part == 0) {  // no visible key: zeros (the reference's l == 0 guard, :103-104)
+      for (int i = threadIdx.x; i < G * D; i += kThreads)
+        store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)(kvh * G + i / D) * p.so_head + i % D, 0.f);
     }
     return;
   }
-  // more partitions than the LDS weight table holds: one pass of max-rescaled sums per output
-  for (int e = threadIdx.x; e < G * D; e += kThreads) {
-    const int g = e / D, d = e % D;
-    const int h = kvh * G + g;
-    const int64_t base = ((int64_t)qi * p.hq + h) * p.max_parts;
-    float m = -INFINITY, l = 0.f, o = 0.f;
-    for (int i = 0; i < arrivals; ++i) {
-      const float mi = ld_dev(&p.ws_ml[(base + i) * 2]);
-      const float li = ld_dev(&p.ws_ml[(base + i) * 2 + 1]);
-      const float ai = ld_dev(&p.ws_acc[(base + i) * D + d]);
-      if (mi == -INFINITY) continue;  // a partition whose keys were all skipped
-      if (mi > m) {
-        const float r = m == -INFINITY ? 0.f : exp2f(m - mi);
-        l *= r;
-        o *= r;
-        m = mi;
-      }
-      const float w = exp2f(mi - m);
-      l = fmaf(w, li, l);
-      o = fmaf(w, ai, o);
+  const int t0 = part * p.part_tokens;
+  const int n = min(qp.kv_len, t0 + p.part_tokens) - t0;
+  const int32_t* bt_row = p.bt + (int64_t)qp.seq * p.sbt;
+
+  // the partition's slice of the block table, validated once, into LDS
+  const int bi0 = t0 / p.block_size;
+  const int nbi = (t0 + n - 1) / p.block_size - bi0 + 1;
+  for (int i = threadIdx.x; i < nbi; i += kThreads) {
+    const int bi = bi0 + i;
+    int blk = bi < p.max_blocks_per_seq ? bt_row[bi] : -1;
+    if (blk < 0 || blk >= p.num_blocks) {
+      blk = -1;
+      if (p.status) atomicOr(p.status, NS_PA_STATUS_BAD_BLOCK);
     }
-    store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
+    s_blk[i] = blk;
   }
+
+  const int c16 = lane & 15, q4 = lane >> 4;
+  // Q^T operand: head c16 (zeros past G), dims 32 s + 8 q4 .. + 7
+  vec qop[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    u32x4 x = {0u, 0u, 0u, 0u};
+    if (c16 < G)
+      x = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.q) + (int64_t)qi * p.sq_tok +
+                                          (int64_t)(kvh * G + c16) * p.sq_head + 32 * s + 8 * q4);
+    qop[s] = __builtin_bit_cast(vec, x);
+  }
+  __syncthreads();
+
+  constexpr int LPR = D / 8;          // lanes (16-byte chunks) of a row
+  constexpr int RPI = 64 / LPR;       // rows of a load instruction
+  constexpr int NL = kStep / RPI;     // load instructions of each kind a step
+  const int row0 = lane / LPR, ch = lane % LPR;
+  const char* kbase = reinterpret_cast<const char*>(p.k) + (int64_t)kvh * p.sk_head * 2;
+  const char* vbase = reinterpret_cast<const char*>(p.v) + (int64_t)kvh * p.sv_head * 2;
+  const int sk_tok = (int)p.sk_tok, sv_tok = (int)p.sv_tok;
+  const uint32_t koff = (uint32_t)(row0 * sk_tok) * 2u + 16u * ch, voff = (uint32_t)(row0 * sv_tok) * 2u + 16u * ch;
+  auto swz = [](int r) -> int {
+    return D == 128 ? ((r & 7) << 1) | ((r >> 3) & 1) : (((r >> 1) & 3) << 1) | ((r >> 3) & 1);
+  };
+  auto slot = [&](int r, int c) -> int { return r * (D * 2) + ((c ^ swz(r)) << 4); };
+  unsigned char* sk = s_kv[wave][0];
+  unsigned char* sv = s_kv[wave][1];
+
+  u32x4 kreg[NL], vreg[NL];
+  uint32_t ok = 0u;      // bit r: row r of the step in the registers is the sequence's
+  int blk[NL], off[NL];
+  auto place_rows = [&](int base) {
+    ok = 0u;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      // the instruction's first row, past the end the last group again; or the lane's own row
+      const int jr = base + RPI * i + (BW ? 0 : row0);
+      const int t = t0 + min(jr, BW ? (n - 1) & -RPI : n - 1);
+      int bi;
+      if (BW || p.bs_shift >= 0) {
+        bi = t >> p.bs_shift;
+        off[i] = t & (p.block_size - 1);
+      } else {
+        bi = t / p.block_size;
+        off[i] = t - bi * p.block_size;
+      }
+      blk[i] = s_blk[bi - bi0];
+      if constexpr (BW) blk[i] = __builtin_amdgcn_readfirstlane(blk[i]);
+      if constexpr (BW) {
+        ok |= blk[i] >= 0 ? ((1u << RPI) - 1u) << (RPI * i) : 0u;
+      } else {
+        const uint64_t good = __ballot(blk[i] >= 0);
+#pragma unroll
+        for (int q = 0; q < RPI; ++q) ok |= (uint32_t)((good >> (q * LPR)) & 1ull) << (RPI * i + q);
+      }
+      if (blk[i] < 0) blk[i] = 0;   // block 0 stands in for an invalid one; its rows are not used
+    }
+    if (n - base < kStep) ok &= n > base ? (1u << (n - base)) - 1u : 0u;
+  };
+  auto load_k = [&]() {
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      kreg[i] = *reinterpret_cast<const u32x4*>(
+          BW ? kbase + ((uint64_t)(uint32_t)blk[i] * (uint32_t)p.sk_blk + (uint32_t)(off[i] * sk_tok)) * 2 + koff
+             : kbase + ((int64_t)blk[i] * p.sk_blk + off[i] * sk_tok) * 2 + 16 * ch);
+  };
+  auto load_v = [&]() {
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      vreg[i] = *reinterpret_cast<const u32x4*>(
+          BW ? vbase + ((uint64_t)(uint32_t)blk[i] * (uint32_t)p.sv_blk + (uint32_t)(off[i] * sv_tok)) * 2 + voff
+             : vbase + ((int64_t)blk[i] * p.sv_blk + off[i] * sv_tok) * 2 + 16 * ch);
+  };
+  auto store_rows = [&](unsigned char* dst, const u32x4 (&x)[NL]) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<u32x4*>(dst + slot(RPI * i + row0, ch)) = x[i];
+  };
+
+  f32x4_t acc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  // The transposing read: lane 16 q + i of a quarter addresses position 4 q + i / 4, dims 4 (i % 4) .. + 3
+  // of the block, and receives positions 4 q .. + 3 of dim i.
+  const int tr_row = 4 * q4 + (c16 >> 2);
+
+  int base = __builtin_amdgcn_readfirstlane(wave) * kStep;
+  if (base < n) {
+    place_rows(base);
+    load_k();
+    __builtin_amdgcn_sched_barrier(0);   // keys first, as in the loop: the first wait is for them alone
+    load_v();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (; base < n; base += kWaves * kStep) {
+    const uint32_t okw = ok;
+    store_rows(sk, kreg);
+    // the next step's rows, past the end the last ones again: loads without a branch around them, so
+    // that the wait for the older ones leaves them in flight
+    place_rows(base + kWaves * kStep);
+    load_k();
+    __builtin_amdgcn_sched_barrier(0);
+    if (okw != kAllOk) {   // weight 0 times a row not of this sequence must be 0
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+        if (!((okw >> (RPI * i + row0)) & 1u)) vreg[i] = u32x4{0u, 0u, 0u, 0u};
+    }
+    store_rows(sv, vreg);
+    load_v();
+    __builtin_amdgcn_wave_barrier();   // the wave's own LDS rows: in order, no workgroup barrier
+    // S^T = K Q^T
+    f32x4_t st[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      st[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const u32x4 x = *reinterpret_cast<const u32x4*>(sk + slot(16 * b + c16, 4 * s + q4));
+        st[b] = M::mma16(__builtin_bit_cast(vec, x), qop[s], st[b]);
+      }
+    }
+
+    // online softmax of head c16 over the step's 32 positions, 8 of them in this lane
+    float mt = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = st[b][i] * p.scale_log2;
+        if (okw != kAllOk && !((okw >> (16 * b + 4 * q4 + i)) & 1u)) x = -INFINITY;
+        st[b][i] = x;
+        mt = fmaxf(mt, x);
+      }
+    mt = fmaxf(mt, __shfl_xor(mt, 16));
+    mt = fmaxf(mt, __shfl_xor(mt, 32));
+    // the reference m moves only for a score more than 8 (log2 units) above it, as in the prefill kernel
+    const bool move = mt > m + 8.f;
+    const float mn = move ? mt : m;
+    const float msub = mn == -INFINITY ? 0.f : mn;
+    if (__ballot(move) != 0ull) {
+      const float alpha = move ? __builtin_amdgcn_exp2f(m - msub) : 1.f;
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[db][i] *= alpha;
+    }
+    m = mn;
+    uint32_t wh[2 * NB], wl[2 * NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i2 = 0; i2 < 2; ++i2) {
+        const float p0 = __builtin_amdgcn_exp2f(st[b][2 * i2] - msub);
+        const float p1 = __builtin_amdgcn_exp2f(st[b][2 * i2 + 1] - msub);
+        l += p0 + p1;
+        const uint32_t hi = M::pack2(p0, p1);
+        wh[2 * b + i2] = hi;
+        wl[2 * b + i2] = M::pack2(p0 - M::lo(hi), p1 - M::hi(hi));
+      }
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      const int c = 2 * db + ((c16 & 3) >> 1);
+      const u32x2 a0 = __builtin_bit_cast(
+          u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                     (__attribute__((address_space(3))) i16x4*)(sv + slot(tr_row, c) + 8 * (c16 & 1))));
+      if constexpr (NB == 1) {
+        acc[db] = M::mma16(a0, u32x2{wh[0], wh[1]}, acc[db]);
+        acc[db] = M::mma16(a0, u32x2{wl[0], wl[1]}, acc[db]);
+      } else {
+        const u32x2 a1 = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                       (__attribute__((address_space(3))) i16x4*)(sv + slot(16 + tr_row, c) + 8 * (c16 & 1))));
+        const vec a = __builtin_bit_cast(vec, (u32x4{a0[0], a0[1], a1[0], a1[1]}));
+        acc[db] = M::mma16(a, __builtin_bit_cast(vec, (u32x4{wh[0], wh[1], wh[2 * NB - 2], wh[2 * NB - 1]})), acc[db]);
+        acc[db] = M::mma16(a, __builtin_bit_cast(vec, (u32x4{wl[0], wl[1], wl[2 * NB - 2], wl[2 * NB - 1]})), acc[db]);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+
+  // the waves' maxima and sums, then their outputs scaled to the common maximum
+  if (q4 == 0 && c16 < G) {
+    s_wm[wave][c16] = m;
+    s_wl[wave][c16] = l;
+  }
+  __syncthreads();
+  float* s_red = reinterpret_cast<float*>(&s_kv[0][0][0]);   // (wave, head, dim); every wave's value rows are read
+  if (c16 < G) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) mx = fmaxf(mx, s_wm[w][c16]);
+    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx);
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s_red[(wave * G + c16) * D + 16 * db + 4 * q4 + i] = acc[db][i] * f;
+    if (wave == 0 && q4 == 0) {
+      float L = 0.f;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w)
+        L = fmaf(s_wm[w][c16] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_wm[w][c16] - mx), s_wl[w][c16], L);
+      s_m[c16] = mx;
+      s_l[c16] = L;
+    }
+  }
+  __syncthreads();
+  finish_partition<T, D, G, kMaxMerge>(p, qi, kvh, part, n_parts,
+                                       [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_red);
 }
 
 // ---- prefill kernel: query tiles on MFMA -------------------------------------------------------
@@ -531,43 +897,6 @@ constexpr int kPfMinPart = 256;
 constexpr int kPfTargetGroups = 512;     // two four-wave workgroups per CU
 constexpr int kPfMinSteps = 4;           // steps a workgroup takes at least when tiles are cut
 static_assert(kPfCols == NS_PA_TILE_COLUMNS, "the header's tile width");
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-
-// The MFMA and the 16-bit type's conversions: pack2 rounds two floats to nearest even into one
-// word (low half the first; v_cvt_pk_bf16_f32 for bfloat16), lo / hi widen a word's halves back.
-template <typename T> struct Mma;
-template <> struct Mma<Bf16> {
-  typedef bf16x8_t vec;
-  static __device__ __forceinline__ f32x16_t mma(vec a, vec b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2_t));
-  }
-  static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
-  static __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-};
-template <> struct Mma<F16> {
-  typedef f16x8_t vec;
-  static __device__ __forceinline__ f32x16_t mma(vec a, vec b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2_t));
-  }
-  static __device__ __forceinline__ float lo(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)w); }
-  static __device__ __forceinline__ float hi(uint32_t w) {
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
-  }
-};
 
 struct PfParams {
   const int32_t* tiles;   // (n_tiles, 3): sequence, first query token (flat index), token count
@@ -1132,15 +1461,23 @@ uint64_t workspace_bytes(int32_t total_q, int32_t hq, int32_t hkv, int32_t head_
 // when f.tiles is set (16-bit types only)
 template <typename T, int D, int G>
 void launch(const PaParams& p, const PfParams& f, int n_tokens, int n_tiles, hipStream_t stream) {
+  // scalar row addresses: power-of-two blocks that hold a wave's load, block strides in 32 bits
+  const bool by_wave = p.bs_shift >= 0 && p.block_size >= 512 / D && p.sk_blk >= 0 && p.sv_blk >= 0 &&
+                       p.sk_blk < INT32_MAX && p.sv_blk < INT32_MAX;
+  (void)by_wave;
   if (n_tokens > 0) {
     dim3 grid(n_tokens, p.hkv, p.max_parts > 0 ? p.max_parts : 1);
-    hipLaunchKernelGGL((pa_partition_kernel<T, D, G>), grid, dim3(kThreads), 0, stream, p);
+    if constexpr (Elem<T>::bytes == 2) {
+      if (by_wave) hipLaunchKernelGGL((pa_decode_kernel<T, D, G, true>), grid, dim3(kThreads), 0, stream, p);
+      else hipLaunchKernelGGL((pa_decode_kernel<T, D, G, false>), grid, dim3(kThreads), 0, stream, p);
+    } else {
+      hipLaunchKernelGGL((pa_partition_kernel<T, D, G>), grid, dim3(kThreads), 0, stream, p);
+    }
   }
   if constexpr (Elem<T>::bytes == 2) {
     if (n_tiles > 0) {
       const dim3 grid((unsigned)(f.grid > 0 ? f.grid : n_tiles * p.hkv));
-      if (p.bs_shift >= 0 && p.block_size >= 512 / D && p.sk_blk >= 0 && p.sv_blk >= 0 && p.sk_blk < INT32_MAX &&
-          p.sv_blk < INT32_MAX)
+      if (by_wave)
         hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, true>), grid, dim3(kPfThreads), 0, stream, p, f);
       else
         hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, false>), grid, dim3(kPfThreads), 0, stream, p, f);

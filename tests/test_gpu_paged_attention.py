@@ -313,3 +313,48 @@ def test_prefill_shared_steps(device, seqs, qlens, scale, bad):
         assert ((a.double() - ref).abs() <= 1e-4 + 2.0 ** -7 * ref.abs()).all()
     else:
         assert_close_to_oracle(a, PA.paged_attention(**oracle_args(case), terms=True), q.dtype)
+
+
+@pytest.mark.parametrize("d,g,dtype,block_size", [(128, 1, torch.bfloat16, 16), (128, 3, torch.float16, 4),
+                                                  (128, 8, torch.bfloat16, 2), (64, 2, torch.float16, 8),
+                                                  (64, 4, torch.bfloat16, 7), (64, 8, torch.float16, 4)])
+def test_decode_step_edges(device, d, g, dtype, block_size):
+    # lengths around a wave's step (16 positions of 128 dims, 32 of 64), the four waves' share and the
+    # partitions; block sizes on both sides of the rule for scalar row addresses
+    lens = [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 257, 1023, 1025, 2500]
+    case = make_case(600 + d + g, lens, [1] * len(lens), hq=2 * g, hkv=2, d=d, dtype=dtype, block_size=block_size)
+    a = check(case, device, max_query_len=1)
+    assert torch.equal(a, run(case, device, max_query_len=1))
+
+
+@pytest.mark.parametrize("num_seqs", [1, 63, 64, 65, 129, 4097])
+def test_decode_token_search(device, num_seqs):
+    # the sequence of a query token is found 64 entries at a time; empty sequences share their start
+    lens = [1 + (7 * i) % 19 for i in range(num_seqs)]
+    qlens = [0 if i % 5 == 3 else 1 for i in range(num_seqs)]
+    case = make_case(700 + num_seqs, lens, qlens, hq=2, hkv=1, d=64, block_size=8)
+    check(case, device, max_query_len=1)
+
+
+def test_decode_invalid_blocks_skip_their_keys(device):
+    # garbage (NaN) in rows that no sequence holds must not reach the outputs
+    case = make_case(800, [300, 40, 2000], [1, 1, 1])
+    free = torch.ones(case["k_cache"].shape[0], dtype=torch.bool)
+    for s, n in enumerate([300, 40, 2000]):
+        free[case["block_tables"][s, :-(-n // 16)].long()] = False
+        last = int(case["block_tables"][s, (n - 1) // 16])
+        if n % 16:
+            case["v_cache"][last, n % 16:] = float("nan")
+            case["k_cache"][last, n % 16:] = float("nan")
+    case["k_cache"][free] = float("nan")
+    case["v_cache"][free] = float("nan")
+    out = run(case, device, max_query_len=1)
+    clean = {k: (torch.nan_to_num(v) if k.endswith("cache") else v) for k, v in case.items()}
+    assert_close_to_oracle(out, PA.paged_attention(**oracle_args(clean), terms=True), case["query"].dtype)
+    bad = {k: (v.clone() if isinstance(v, torch.Tensor) else v) for k, v in clean.items()}
+    bad["block_tables"][0, 3] = -1
+    bad["block_tables"][2, 5:9] = 10 ** 6
+    a = run(bad, device, max_query_len=1)
+    f32 = {k: (v.float() if isinstance(v, torch.Tensor) and v.is_floating_point() else v) for k, v in bad.items()}
+    ref = run(f32, device, max_query_len=1).double()
+    assert ((a.double() - ref).abs() <= 1e-4 + 2.0 ** -7 * ref.abs()).all()
