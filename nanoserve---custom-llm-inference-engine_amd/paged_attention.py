@@ -210,15 +210,20 @@ class PagedAttentionPlan:
 def _dtype_code(dtype) -> int:
     import torch
 
-    codes = {torch.float32: NS_PA_DTYPE_F32, torch.bfloat16: NS_PA_DTYPE_BF16, torch.float16: NS_PA_DTYPE_F16}
-    if dtype not in codes:
-        raise PagedAttentionError(f"unsupported dtype {dtype} (float32, bfloat16, float16)")
-    return codes[dtype]
+    if dtype is torch.bfloat16:
+        return NS_PA_DTYPE_BF16
+    if dtype is torch.float16:
+        return NS_PA_DTYPE_F16
+    if dtype is torch.float32:
+        return NS_PA_DTYPE_F32
+    raise PagedAttentionError(f"unsupported dtype {dtype} (float32, bfloat16, float16)")
 
 
 def _i32(t, device):
     import torch
 
+    if t.dtype is torch.int32 and t.device == device and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.int32).contiguous()
 
 
@@ -249,6 +254,10 @@ def paged_attention_hip(query, k_cache, v_cache, block_tables, seq_lens, query_s
         raise PagedAttentionError("paged_attention_hip needs device tensors")
     if stream is None:
         s = torch.cuda.current_stream(dev)
+        if dev.index == torch.cuda.current_device():   # already where the call goes: no stream to switch to and back
+            return _paged_attention_on(lib, s, query, k_cache, v_cache, block_tables, seq_lens, query_start_loc,
+                                       query_lens, scale, block_size, max_seq_len, max_query_len, plan, out,
+                                       workspace, counters, status)
     elif isinstance(stream, torch.cuda.Stream):
         s = stream
     elif int(stream) == 0:
@@ -271,18 +280,20 @@ def _paged_attention_on(lib, s, query, k_cache, v_cache, block_tables, seq_lens,
 
     dev = query.device
     total_q, hq, d = query.shape
-    nb, bs, hkv, dk = k_cache.shape
-    if v_cache.shape != k_cache.shape or dk != d:
+    nb, bs, hkv, dk = k_shape = k_cache.shape
+    dtype = query.dtype
+    if v_cache.shape != k_shape or dk != d:
         raise PagedAttentionError(f"cache shapes {tuple(k_cache.shape)}, {tuple(v_cache.shape)} do not match "
                                   f"the query's head_dim {d}")
-    if k_cache.dtype != query.dtype or v_cache.dtype != query.dtype:
+    if k_cache.dtype != dtype or v_cache.dtype != dtype:
         raise PagedAttentionError("query and caches must share one dtype")
     if bs != block_size:
         raise PagedAttentionError(f"block_size {block_size} != the cache's {bs}")
     if total_q == 0:  # nothing to attend (an empty tensor's strides are arbitrary)
         return torch.empty_like(query) if out is None else out
-    for name, t in (("query", query), ("k_cache", k_cache), ("v_cache", v_cache)):
-        if t.stride(-1) != 1:
+    q_stride, k_stride, v_stride = query.stride(), k_cache.stride(), v_cache.stride()
+    for name, stride in (("query", q_stride), ("k_cache", k_stride), ("v_cache", v_stride)):
+        if stride[-1] != 1:
             raise PagedAttentionError(f"{name} must have a unit head_dim stride")
     bt = _i32(block_tables, dev)
     sl = _i32(seq_lens, dev)
@@ -308,21 +319,24 @@ def _paged_attention_on(lib, s, query, k_cache, v_cache, block_tables, seq_lens,
         max_seq_len = int(sl.max().item()) if num_seqs else 0
     if out is None:
         out = torch.empty_like(query)
+        o_stride = out.stride()
     elif out.shape != query.shape or out.dtype != query.dtype or out.device != dev:
         raise PagedAttentionError("out must match query's shape, dtype and device")
     elif out.stride(-1) != 1:
         raise PagedAttentionError("out must have a unit head_dim stride")
+    else:
+        o_stride = out.stride()
     if status is not None and (status.dtype != torch.int32 or status.device != dev or status.numel() < 1):
         raise PagedAttentionError("status must be an int32 device tensor")
     a = NsPagedAttnArgs(
         query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), bt.data_ptr(), sl.data_ptr(),
         qsl.data_ptr(), ql.data_ptr(), status.data_ptr() if status is not None else None,
         None, 0, None,
-        query.stride(0), query.stride(1), k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
-        v_cache.stride(0), v_cache.stride(1), v_cache.stride(2), out.stride(0), out.stride(1),
+        q_stride[0], q_stride[1], k_stride[0], k_stride[1], k_stride[2],
+        v_stride[0], v_stride[1], v_stride[2], o_stride[0], o_stride[1],
         bt.stride(0) if bt.dim() == 2 else 0,
         total_q, num_seqs, hq, hkv, d, bs, nb, bt.shape[1] if bt.dim() == 2 else 0, max_seq_len,
-        _dtype_code(query.dtype), float(scale))
+        _dtype_code(dtype), float(scale))
     if tiles is not None:
         a.decode_tokens, a.n_decode_tokens = tokens
         a.prefill_tiles, a.n_prefill_tiles = tiles
