@@ -286,7 +286,7 @@ __device__ __forceinline__ void lm_load_lds16(__amdgpu_buffer_rsrc_t r, unsigned
 
 // Large batches (more than 64 rows) over the packed weight: the column-owner form.  Wave w owns vocab rows
 // n0 + 32 w .. + 31 and all MT = 32 TM batch rows of the workgroup (TM tiles of 32 x 32,
-// 16 TM accumulators per lane), so each weight piece is used by one wave only: it goes from
+// 16 TM accumulators per lane; TM = 4, 6, 8 or 10), so each weight piece is used by one wave only: it goes from
 // HBM straight into that wave's B operand registers and never through LDS.  A register set
 // holds one stage (four k-steps); each k-step's registers are refilled with the stage three
 // ahead as soon as its products are issued, so about three stages of weight (96 KB per CU)

@@ -137,3 +137,15 @@ def test_packed_large_batch_gathers_rows_and_flags_bad_indices(device, m):
     good = ~bad
     check(out[good], hidden_full, weight, rows=rows[good])
     assert torch.equal(out[good].contiguous().view(torch.int16), plain[good].contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("m", [65, 128, 129, 192, 193, 257, 320, 321, 385, 641])
+def test_packed_batch_row_tiles(device, m):
+    """Every height of the column-owner kernel's workgroup rows (128, 192, 256, 320) at its edges, one
+    to three of them: the same bits as the weight as stored."""
+    hidden, weight = make(device, m, 517, 256, seed=57 + m, scale=2.0)
+    packed = L.lm_head_bf16(hidden, L.PackedLmHead(weight))
+    plain = L.lm_head_bf16(hidden, weight)
+    torch.cuda.synchronize()
+    check(packed, hidden, weight)
+    assert torch.equal(packed.view(torch.int16), plain.view(torch.int16))
