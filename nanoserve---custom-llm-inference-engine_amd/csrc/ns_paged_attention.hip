@@ -1590,7 +1590,9 @@ int ns_paged_attention(const ns_paged_attn_args* a, hipStream_t stream) {
   p.qsl = a->query_start_loc;
   p.qlens = a->query_lens;
   p.status = a->status;
-  p.ws_acc = reinterpret_cast<float*>(a->workspace);
+  // no room of its own (the workspace may still be there for the tiles): a row longer than max_seq_len
+  // allows is flagged and leaves no partials
+  p.ws_acc = need ? reinterpret_cast<float*>(a->workspace) : nullptr;
   p.ws_ml = need ? p.ws_acc + (uint64_t)a->total_q * a->num_heads_q * max_parts * a->head_dim : nullptr;
   p.counters = a->counters;
   p.sq_tok = a->stride_q_token;

@@ -358,3 +358,18 @@ def test_decode_invalid_blocks_skip_their_keys(device):
     f32 = {k: (v.float() if isinstance(v, torch.Tensor) and v.is_floating_point() else v) for k, v in bad.items()}
     ref = run(f32, device, max_query_len=1).double()
     assert ((a.double() - ref).abs() <= 1e-4 + 2.0 ** -7 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_long_decode_row_beside_cut_tiles(device, dtype):
+    # 130 listed tokens of 8 KV heads at max_seq_len 1000 fit one partition each and need no workspace,
+    # the tile beside them is cut and does.  A decode row longer than max_seq_len allows is flagged, its
+    # output undefined; nothing of it reaches the tile's partials, and all other rows are exact
+    seqs, qlens = [990] + [40] * 129 + [1500], [30] + [1] * 130
+    case = make_case(810, seqs, qlens, hq=8, hkv=8, d=64, dtype=dtype)
+    assert A.workspace_bytes(130, 8, 8, 64, 1000) == 0
+    status = torch.zeros(1, dtype=torch.int32, device=device)
+    out = run(case, device, max_seq_len=1000, status=status)
+    assert status.item() == A.STATUS_SEQ_TOO_LONG
+    ref, cond = PA.paged_attention(**oracle_args(case), terms=True)
+    assert_close_to_oracle(out[:-1], (ref[:-1], cond[:-1]), dtype)
