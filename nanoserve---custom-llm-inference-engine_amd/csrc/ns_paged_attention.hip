@@ -36,6 +36,11 @@ constexpr int kWaves = kThreads / 64;
 constexpr int kSub = 2;                 // KV positions per lane per batch
 constexpr int kMaxPart = 1024;          // largest KV partition (LDS score buffer)
 constexpr int kMinPart = 64;
+// partitions of a row merged through a table of their weights in LDS (one long row of few KV heads has
+// hundreds): the loop that takes more reads three words per partition and output one after the other.
+// one row of 17000 .. 65536 positions, 1 .. 3 KV heads (266 .. 1024 partitions, bf16, head_dim 128,
+// G = 1 .. 8): 29-296 us with the table, 75-1145 by the loop
+constexpr int kMaxMerge = 1024;
 constexpr int kTargetGroups = 1024;     // workgroups a launch aims for before splitting stops
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -280,7 +285,7 @@ template <> struct Mma<F16> {
 // The end of a partition: the sum over the waves of red(wave, head, dim), s_m and s_l the partition's
 // maximum (log2 units) and sum of weights per head.  s_w: G * kMaxMerge floats of LDS, free once red
 // has been read.
-template <typename T, int D, int G, int kMaxMerge, typename Red>
+template <typename T, int D, int G, typename Red>
 __device__ __forceinline__ void finish_partition(const PaParams& p, int qi, int kvh, int part, int n_parts, Red red,
                                                  float* s_m, float* s_l, float* s_w) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -385,6 +390,7 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   constexpr int NSLOT = 64 / L;       // positions a wave covers per row of a batch
   constexpr int kBatch = NSLOT * kSub;  // KV positions per wave batch
   static_assert(G <= L, "the lane with dl == g stores head g's score");
+  static_assert(kMaxMerge <= kMaxPart, "s_score becomes the merge's weight table");
   __shared__ float s_score[G * kMaxPart];
   __shared__ float s_red[kWaves * G * D];
   __shared__ float s_m[G], s_l[G];
@@ -556,7 +562,7 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   }
   __syncthreads();
 
-  finish_partition<T, D, G, kMaxPart>(p, qi, kvh, part, n_parts,
+  finish_partition<T, D, G>(p, qi, kvh, part, n_parts,
                                       [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_score);
 }
 
@@ -595,7 +601,6 @@ __global__ __launch_bounds__(kThreads)
   constexpr int NB = D == 128 ? 1 : 2;  // 16-row blocks of a wave's step
   constexpr int kStep = 16 * NB;        // its positions
   constexpr uint32_t kAllOk = NB == 1 ? 0xffffu : 0xffffffffu;
-  constexpr int kMaxMerge = kMaxPart / 4;
   static_assert(G <= 16, "the heads are the 16 columns");
   __shared__ __align__(16) unsigned char s_kv[kWaves][2][kStep * D * 2];   // then the waves' outputs, then merge weights
   __shared__ float s_wm[kWaves][G], s_wl[kWaves][G];
@@ -847,7 +852,7 @@ __global__ __launch_bounds__(kThreads)
     }
   }
   __syncthreads();
-  finish_partition<T, D, G, kMaxMerge>(p, qi, kvh, part, n_parts,
+  finish_partition<T, D, G>(p, qi, kvh, part, n_parts,
                                        [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_red);
 }
 

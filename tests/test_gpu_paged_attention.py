@@ -145,6 +145,17 @@ def test_more_partitions_than_the_lds_weight_table(device):
     check(case, device)
 
 
+@pytest.mark.parametrize("ctx,parts", [(16384, 256), (16385, 257), (40000, 625), (65536, 1024), (65600, 1025)])
+@pytest.mark.parametrize("hq,d,dtype", [(8, 128, torch.bfloat16), (4, 64, torch.float16)])
+def test_one_long_row_of_few_kv_heads(device, ctx, parts, hq, d, dtype):
+    # a row of one KV head merges hundreds of partitions: through the LDS weight table up to 1024 of
+    # them, whatever the number of heads it is shared by, and past it by the one-pass loop
+    case = make_case(900 + parts, [ctx], [1], hq=hq, hkv=1, d=d, dtype=dtype)
+    assert A.workspace_bytes(1, hq, 1, d, ctx) == hq * parts * (d + 2) * 4
+    a = check(case, device, max_query_len=1)
+    assert torch.equal(a, run(case, device, max_query_len=1))
+
+
 def test_side_stream_and_output_stride(device):
     """A call on a side stream (its temporaries and counters made on that stream) equals the
     call on the current stream bit for bit; an output whose head_dim stride is not 1 is refused
