@@ -284,28 +284,44 @@ template <> struct Mma<F16> {
 
 // The end of a partition: the sum over the waves of red(wave, head, dim), s_m and s_l the partition's
 // maximum (log2 units) and sum of weights per head.  s_w: G * kMaxMerge floats of LDS, free once red
-// has been read.
-template <typename T, int D, int G, typename Red>
+// has been read.  s_odd (or NULL): an LDS word, 0 so far; with a sum that is NaN, infinite or large enough
+// to overflow in the merge, redo() makes red, s_m and s_l anew and they are stored again.
+template <typename T, int D, int G, typename Red, typename Redo>
 __device__ __forceinline__ void finish_partition(const PaParams& p, int qi, int kvh, int part, int n_parts, Red red,
-                                                 float* s_m, float* s_l, float* s_w) {
+                                                 float* s_m, float* s_l, float* s_w, int* s_odd, Redo redo) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const bool direct = n_parts == 1;
-  for (int e = threadIdx.x; e < G * D; e += kThreads) {
-    const int g = e / D, d = e % D;
-    float o = 0.f;
+  auto store = [&]() -> bool {
+    bool odd = false;
+    for (int e = threadIdx.x; e < G * D; e += kThreads) {
+      const int g = e / D, d = e % D;
+      float o = 0.f;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) o += red(w, g, d);
-    const int h = kvh * G + g;
-    if (direct) {
-      const float l = s_l[g];
-      store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
-    } else if (p.ws_acc && part < p.max_parts) {
-      const int64_t slot_idx = ((int64_t)qi * p.hq + h) * p.max_parts + part;
-      st_dev(&p.ws_acc[slot_idx * D + d], o);
-      if (d == 0) {
-        st_dev(&p.ws_ml[slot_idx * 2], s_m[g]);
-        st_dev(&p.ws_ml[slot_idx * 2 + 1], s_l[g]);
+      for (int w = 0; w < kWaves; ++w) o += red(w, g, d);
+      odd |= !(fabsf(o) < 0x1p100f);
+      const int h = kvh * G + g;
+      if (direct) {
+        const float l = s_l[g];
+        store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
+      } else if (p.ws_acc && part < p.max_parts) {
+        const int64_t slot_idx = ((int64_t)qi * p.hq + h) * p.max_parts + part;
+        st_dev(&p.ws_acc[slot_idx * D + d], o);
+        if (d == 0) {
+          st_dev(&p.ws_ml[slot_idx * 2], s_m[g]);
+          st_dev(&p.ws_ml[slot_idx * 2 + 1], s_l[g]);
+        }
       }
+    }
+    return odd;
+  };
+  const bool odd = store();
+  if (s_odd != nullptr) {
+    if (odd) *s_odd = 1;
+    __syncthreads();
+    if (__builtin_expect(*s_odd != 0, 0)) {
+      redo();
+      __syncthreads();
+      store();
     }
   }
   if (direct || !p.ws_acc || part >= p.max_parts) return;
@@ -563,7 +579,84 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   __syncthreads();
 
   finish_partition<T, D, G>(p, qi, kvh, part, n_parts,
-                                      [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_score);
+                            [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_score,
+                            nullptr, []() {});
+}
+
+// A partition in float arithmetic throughout, as the float32 kernel computes it: what pa_decode_kernel
+// falls back to when its sums are not finite, or near it.  The two 16-bit parts of a weight times an
+// infinite value are NaN where the weight itself gives infinity (0 * inf for a low part of 0, inf - inf
+// for a negative one), and its weights of up to 2^8 can overflow on values near bfloat16's largest.  One thread per
+// score and per output, rows read element by element: a partition of 1024 positions takes some hundred
+// microseconds, on such values alone.  Leaves the sums in s_buf as (wave, head, dim), all in wave 0.
+template <typename T, int D, int G>
+__device__ __forceinline__ void plain_partition(const PaParams& p, int qi, int kvh, int t0, int n, const int* s_blk,
+                                                float* s_buf, float* s_m, float* s_l) {
+  using M = Mma<T>;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int bi0 = t0 / p.block_size;
+  auto words = [](const void* base, int64_t elem) -> const uint32_t* {   // of a row, 16-byte aligned
+    return reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(base) + elem);
+  };
+  for (int e = threadIdx.x; e < G * n; e += kThreads) {
+    const int g = e / n, j = e - g * n;
+    const int bi = (t0 + j) / p.block_size, off = t0 + j - bi * p.block_size;
+    const int blk = s_blk[bi - bi0];
+    float sc = -INFINITY;
+    if (blk >= 0) {
+      const uint32_t* q = words(p.q, (int64_t)qi * p.sq_tok + (int64_t)(kvh * G + g) * p.sq_head);
+      const uint32_t* k = words(p.k, (int64_t)blk * p.sk_blk + (int64_t)off * p.sk_tok + (int64_t)kvh * p.sk_head);
+      sc = 0.f;
+      for (int i = 0; i < D / 2; ++i) {
+        sc = fmaf(M::lo(q[i]) * p.scale_log2, M::lo(k[i]), sc);
+        sc = fmaf(M::hi(q[i]) * p.scale_log2, M::hi(k[i]), sc);
+      }
+    }
+    s_buf[g * kMaxPart + j] = sc;
+  }
+  __syncthreads();
+  for (int g = wave; g < G; g += kWaves) {
+    float m = -INFINITY, l = 0.f;
+    for (int j = lane; j < n; j += 64) m = fmaxf(m, s_buf[g * kMaxPart + j]);
+    m = wave_max(m);
+    for (int j = lane; j < n; j += 64) {
+      const float w = m == -INFINITY ? 0.f : exp2f(s_buf[g * kMaxPart + j] - m);
+      s_buf[g * kMaxPart + j] = w;
+      l += w;
+    }
+    l = wave_sum(l);
+    if (lane == 0) {
+      s_m[g] = m;
+      s_l[g] = l;
+    }
+  }
+  __syncthreads();
+  constexpr int NE = (G * D + kThreads - 1) / kThreads;   // outputs per thread
+  float o[NE];
+#pragma unroll
+  for (int r = 0; r < NE; ++r) {
+    const int e = (int)threadIdx.x + r * kThreads;
+    o[r] = 0.f;
+    if (e >= G * D) continue;
+    const int g = e / D, d = e % D;
+    for (int j = 0; j < n; ++j) {
+      const int bi = (t0 + j) / p.block_size, off = t0 + j - bi * p.block_size;
+      const int blk = s_blk[bi - bi0];
+      if (blk < 0) continue;
+      const uint32_t w =
+          words(p.v, (int64_t)blk * p.sv_blk + (int64_t)off * p.sv_tok + (int64_t)kvh * p.sv_head)[d >> 1];
+      o[r] = fmaf(s_buf[g * kMaxPart + j], d & 1 ? M::hi(w) : M::lo(w), o[r]);
+    }
+  }
+  __syncthreads();   // the weights are read
+#pragma unroll
+  for (int r = 0; r < NE; ++r) {
+    const int e = (int)threadIdx.x + r * kThreads;
+    if (e >= G * D) continue;
+    s_buf[e] = o[r];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) s_buf[w * G * D + e] = 0.f;
+  }
 }
 
 // The 16-bit types' partition kernel: the same workgroups, partitions, partials and merge, with the
@@ -604,9 +697,11 @@ __global__ __launch_bounds__(kThreads)
   static_assert(G <= 16, "the heads are the 16 columns");
   __shared__ __align__(16) unsigned char s_kv[kWaves][2][kStep * D * 2];   // then the waves' outputs, then merge weights
   __shared__ float s_wm[kWaves][G], s_wl[kWaves][G];
+  __shared__ int s_odd;   // a sum is not finite, or near it
   __shared__ float s_m[G], s_l[G];
   __shared__ int s_blk[kMaxPart + 2];   // physical block of each block-table entry the partition spans
-  static_assert(sizeof(s_kv) >= (size_t)kWaves * G * D * 4 && sizeof(s_kv) >= (size_t)G * kMaxMerge * 4, "reuse");
+  static_assert(sizeof(s_kv) >= (size_t)kWaves * G * D * 4 && sizeof(s_kv) >= (size_t)G * kMaxMerge * 4 &&
+                    sizeof(s_kv) >= (size_t)G * kMaxPart * 4, "reuse");
 
   const int qi = p.tokens != nullptr ? p.tokens[blockIdx.x] : (int)blockIdx.x;
   const int kvh = blockIdx.y, part = blockIdx.z;
@@ -642,6 +737,7 @@ __global__ __launch_bounds__(kThreads)
     }
     s_blk[i] = blk;
   }
+  if (threadIdx.x == 0) s_odd = 0;
 
   const int c16 = lane & 15, q4 = lane >> 4;
   // Q^T operand: head c16 (zeros past G), dims 32 s + 8 q4 .. + 7
@@ -852,8 +948,9 @@ __global__ __launch_bounds__(kThreads)
     }
   }
   __syncthreads();
-  finish_partition<T, D, G>(p, qi, kvh, part, n_parts,
-                                       [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_red);
+  finish_partition<T, D, G>(p, qi, kvh, part, n_parts, [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; },
+                            s_m, s_l, s_red, &s_odd,
+                            [&]() { plain_partition<T, D, G>(p, qi, kvh, t0, n, s_blk, s_red, s_m, s_l); });
 }
 
 // ---- prefill kernel: query tiles on MFMA -------------------------------------------------------

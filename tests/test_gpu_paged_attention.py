@@ -384,3 +384,31 @@ def test_long_decode_row_beside_cut_tiles(device, dtype):
     assert status.item() == A.STATUS_SEQ_TOO_LONG
     ref, cond = PA.paged_attention(**oracle_args(case), terms=True)
     assert_close_to_oracle(out[:-1], (ref[:-1], cond[:-1]), dtype)
+
+
+@pytest.mark.parametrize("g,d,dtype", [(3, 128, torch.bfloat16), (8, 128, torch.float16), (4, 64, torch.bfloat16),
+                                       (1, 64, torch.float16), (1, 128, torch.float32)])
+def test_decode_values_that_are_not_finite(device, g, d, dtype):
+    # infinities, NaN and values near the type's largest in visible rows, in whole and in split rows: each
+    # reaches its own output element as in float arithmetic (weight times infinity is infinity), no other
+    lens = [1, 40, 300, 700, 2500]
+    case = make_case(820 + d + g, lens, [1] * 5, hq=2 * g, hkv=2, d=d, dtype=dtype)
+    v, bt = case["v_cache"], case["block_tables"]
+
+    def put(s, t, head, dim, x):
+        v[int(bt[s, t // 16]), t % 16, head, dim] = x
+
+    for s, n in enumerate(lens):
+        put(s, n - 1, 0, 3, float("inf"))
+        put(s, n // 2, 1, 5, float("-inf"))
+        put(s, n // 3, 0, 8, float("nan"))
+        put(s, n - 1, 1, 11, torch.finfo(dtype).max)   # the largest value, at a weight of at most 1
+    for s, n in enumerate(lens[1:], 1):
+        put(s, 0, 1, 17, float("inf"))                 # both infinities: NaN
+        put(s, n - 2, 1, 17, float("-inf"))
+    out = run(case, device, max_query_len=1)
+    ref, cond = PA.paged_attention(**oracle_args(case), terms=True)
+    got, odd = out.double().cpu().numpy(), ~np.isfinite(ref)
+    assert odd.any() and np.array_equal(got[odd], ref[odd], equal_nan=True)
+    fine = torch.from_numpy(np.where(odd, 0.0, got))
+    assert_close_to_oracle(fine, (np.where(odd, 0.0, ref), np.where(odd, 0.0, cond)), dtype)
