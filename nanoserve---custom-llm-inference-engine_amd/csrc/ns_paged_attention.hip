@@ -240,9 +240,19 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 // The MFMA and the 16-bit type's conversions: pack2 rounds two floats to nearest even into one
 // word (low half the first; v_cvt_pk_bf16_f32 for bfloat16), lo / hi widen a word's halves back.
+//
+// A weight 2^(score - m) enters the value product as a high and a low 16-bit part.  m follows a column's
+// largest score: it moves when a score exceeds it by more than kLift + kGap (log2 units), then to kLift
+// below that score, so that the largest weight lies in [2^kLift, 2^(kLift + kGap)].  bfloat16 has
+// float32's exponents: both parts of every weight keep their bits, and m moves rarely.  float16 ends at
+// 2^-24: the weights are lifted to just below its largest value, so that those far below a column's
+// largest are not lost; where kLowScale is used the low part is a multiple larger too, and the sum of its
+// products is divided by it.  A weight w relative to the largest then carries an absolute error of at
+// most 2^-(25 + kLift) (2^-(36 + kLift) with kLowScale) besides the 2^-22 (bfloat16: 2^-17) relative one.
 template <typename T> struct Mma;
 template <> struct Mma<Bf16> {
   typedef bf16x8_t vec;
+  static constexpr float kGap = 8.f, kLift = 0.f, kLowScale = 1.f;
   static __device__ __forceinline__ f32x4_t mma16(vec a, vec b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -261,6 +271,7 @@ template <> struct Mma<Bf16> {
 };
 template <> struct Mma<F16> {
   typedef f16x8_t vec;
+  static constexpr float kGap = 2.f, kLift = 13.f, kLowScale = 2048.f;
   static __device__ __forceinline__ f32x4_t mma16(vec a, vec b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -674,8 +685,9 @@ __device__ __forceinline__ void plain_partition(const PaParams& p, int qi, int k
 //   * S^T: lane l holds head l % 16 at positions 16 b + 4 (l / 16) + i of row block b.  Its weights are
 //     the B operand of O^T += V^T P^T as they are, with k-slot i of quarter l / 16 at position
 //     4 (l / 16) + i for i < 4, else 12 + 4 (l / 16) + i; the V^T operand is read in that order by two
-//     transposing reads from the wave's own LDS rows.  P goes in as a high and a low 16-bit part, as in
-//     the prefill kernel.
+//     transposing reads from the wave's own LDS rows.  P goes in as a high and a low 16-bit part (Mma);
+//     float16's low parts are summed apart and scaled back (64 rows of up to 2048, 128 dims: 60.3 us
+//     without, 61.5 with).
 //   * LDS rows are unpadded; 16-byte chunk c of row r sits at c ^ swz(r), under which the 16 rows of a
 //     write and the 8 rows of a transposing read hit the 64 banks once.
 // Bound by HBM.  Measured (bf16, 8 KV heads of 128 dims, blocks of 16; the vector form, then this):
@@ -874,9 +886,9 @@ __global__ __launch_bounds__(kThreads)
       }
     mt = fmaxf(mt, __shfl_xor(mt, 16));
     mt = fmaxf(mt, __shfl_xor(mt, 32));
-    // the reference m moves only for a score more than 8 (log2 units) above it, as in the prefill kernel
-    const bool move = mt > m + 8.f;
-    const float mn = move ? mt : m;
+    // the reference m moves only for a score well above it (Mma)
+    const bool move = mt > m + (M::kLift + M::kGap);
+    const float mn = move ? mt - M::kLift : m;
     const float msub = mn == -INFINITY ? 0.f : mn;
     if (__ballot(move) != 0ull) {
       const float alpha = move ? __builtin_amdgcn_exp2f(m - msub) : 1.f;
@@ -897,8 +909,18 @@ __global__ __launch_bounds__(kThreads)
         l += p0 + p1;
         const uint32_t hi = M::pack2(p0, p1);
         wh[2 * b + i2] = hi;
-        wl[2 * b + i2] = M::pack2(p0 - M::lo(hi), p1 - M::hi(hi));
+        wl[2 * b + i2] = M::pack2((p0 - M::lo(hi)) * M::kLowScale, (p1 - M::hi(hi)) * M::kLowScale);
       }
+    // the low parts' products, added to the sum, or by themselves and scaled back
+    auto add_low = [&](auto a, auto w, f32x4_t& sum) {
+      if constexpr (M::kLowScale == 1.f) {
+        sum = M::mma16(a, w, sum);
+      } else {
+        const f32x4_t t = M::mma16(a, w, f32x4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] = fmaf(t[i], 1.f / M::kLowScale, sum[i]);
+      }
+    };
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
       const int c = 2 * db + ((c16 & 3) >> 1);
@@ -907,14 +929,14 @@ __global__ __launch_bounds__(kThreads)
                      (__attribute__((address_space(3))) i16x4*)(sv + slot(tr_row, c) + 8 * (c16 & 1))));
       if constexpr (NB == 1) {
         acc[db] = M::mma16(a0, u32x2{wh[0], wh[1]}, acc[db]);
-        acc[db] = M::mma16(a0, u32x2{wl[0], wl[1]}, acc[db]);
+        add_low(a0, u32x2{wl[0], wl[1]}, acc[db]);
       } else {
         const u32x2 a1 = __builtin_bit_cast(
             u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                        (__attribute__((address_space(3))) i16x4*)(sv + slot(16 + tr_row, c) + 8 * (c16 & 1))));
         const vec a = __builtin_bit_cast(vec, (u32x4{a0[0], a0[1], a1[0], a1[1]}));
         acc[db] = M::mma16(a, __builtin_bit_cast(vec, (u32x4{wh[0], wh[1], wh[2 * NB - 2], wh[2 * NB - 1]})), acc[db]);
-        acc[db] = M::mma16(a, __builtin_bit_cast(vec, (u32x4{wl[0], wl[1], wl[2 * NB - 2], wl[2 * NB - 1]})), acc[db]);
+        add_low(a, __builtin_bit_cast(vec, (u32x4{wl[0], wl[1], wl[2 * NB - 2], wl[2 * NB - 1]})), acc[db]);
       }
     }
     __builtin_amdgcn_wave_barrier();

@@ -412,3 +412,29 @@ def test_decode_values_that_are_not_finite(device, g, d, dtype):
     assert odd.any() and np.array_equal(got[odd], ref[odd], equal_nan=True)
     fine = torch.from_numpy(np.where(odd, 0.0, got))
     assert_close_to_oracle(fine, (np.where(odd, 0.0, ref), np.where(odd, 0.0, cond)), dtype)
+
+
+def sink_case(seed, seq_lens, query_lens, below, sinks, hq, hkv, d, dtype):
+    """Keys of the positions ``sinks`` outweigh all others by about 2 ** below and their values are 0 (an
+    attention sink), so that an output is the sum of the others' small weights; their values are about 256."""
+    case = make_case(seed, seq_lens, query_lens, hq=hq, hkv=hkv, d=d, dtype=dtype)
+    rng = torch.Generator().manual_seed(seed)
+    k, v, bt = case["k_cache"], case["v_cache"], case["block_tables"]
+    case["query"].fill_(1.0)
+    k.copy_(torch.randn(k.shape, generator=rng) * 0.3)
+    v.copy_((torch.rand(v.shape, generator=rng) + 0.5) * 256)
+    for s, n in enumerate(seq_lens):
+        for t in sinks:
+            if t < n:
+                k[int(bt[s, t // 16]), t % 16] = below * np.log(2.0) / np.sqrt(d)
+                v[int(bt[s, t // 16]), t % 16] = 0.0
+    return case
+
+
+@pytest.mark.parametrize("below", [10, 18, 22, 24.5, 27, 31, 35])
+@pytest.mark.parametrize("d,dtype", [(64, torch.float16), (128, torch.float16), (128, torch.bfloat16)])
+def test_decode_small_weights_beside_large_ones(device, below, d, dtype):
+    # in whole rows (partitions of 1024 positions) every wave has a sink, in split ones the first has
+    lens = [1024, 700, 64, 17] * 32
+    check(sink_case(830, lens, [1] * 128, below, (0, 16, 32, 48, 64, 96), 8, 8, d, dtype), device, max_query_len=1)
+    check(sink_case(831, [3000, 200], [1, 1], below, (0,), 6, 2, d, dtype), device, max_query_len=1)
