@@ -993,9 +993,10 @@ __global__ __launch_bounds__(kThreads)
 //     from the S^T layout as the B operand: k-slot i of the lanes of half h is position
 //     16 s + 8 (i / 4) + 4 h + i % 4 of the step, and the V^T operand is read in that order from
 //     the transposed value rows (two 8-byte reads).  P goes in as two 16-bit parts, hi = RN(p)
-//     and lo = RN(p - hi): both products with a value are exact in float32, so the sum carries p
-//     to about 2^-17 relative, the float32 arithmetic of the reference's kernel (a single 16-bit
-//     P would round each weight by up to 2^-9).
+//     and lo = RN(p - hi), whose products with a value are exact in float32: bfloat16 carries p to
+//     about 2^-17 relative, float16 to 2^-22 and 2^-38 of the column's largest weight (Mma; its low
+//     parts summed apart, as in the decode kernel, took 5 to 9% more), where a single 16-bit P
+//     would round each weight by up to 2^-9.
 // The scores are the float32 dot products times scale * log2(e) (folded into the exponent's fma)
 // and exp2 replaces exp, as in the decode kernel.
 //
@@ -1370,12 +1371,11 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
           for (int e = 0; e < 16; ++e) mt = fmaxf(mt, st[rb][e]);
         mt = fmaxf(mt, __shfl_xor(mt, 32)) * scale;
-        // The column's reference m moves only when a score exceeds it by more than 8 (log2 units),
-        // to the new maximum: weights stay at most 2^8 and the accumulators are rescaled rarely.
-        // exp2 by v_exp_f32 (a weight below 2^-126 flushes to zero); -inf scores weigh 0, and a
-        // column with no score yet subtracts 0.
-        const bool move = mt > m + 8.f;
-        const float mn = move ? mt : m;
+        // The column's reference m moves only for a score well above it (Mma): the accumulators are
+        // rescaled rarely.  exp2 by v_exp_f32 (a weight below 2^-126 flushes to zero); -inf scores weigh 0,
+        // and a column with no score yet subtracts 0.
+        const bool move = mt > m + (M::kLift + M::kGap);
+        const float mn = move ? mt - M::kLift : m;
         const float msub = mn == -INFINITY ? 0.f : mn;
         const float alpha = move ? __builtin_amdgcn_exp2f(m - msub) : 1.f;
         m = mn;

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from conftest import pkg
-from pa_cases import assert_close_to_oracle, make_case, oracle_args, to_device
+from pa_cases import ARITH_K, UNIT, assert_close_to_oracle, make_case, oracle_args, to_device
 from oracle import paged_attention_oracle as PA
 
 pytestmark = pytest.mark.gpu
@@ -438,3 +438,17 @@ def test_decode_small_weights_beside_large_ones(device, below, d, dtype):
     lens = [1024, 700, 64, 17] * 32
     check(sink_case(830, lens, [1] * 128, below, (0, 16, 32, 48, 64, 96), 8, 8, d, dtype), device, max_query_len=1)
     check(sink_case(831, [3000, 200], [1, 1], below, (0,), 6, 2, d, dtype), device, max_query_len=1)
+
+
+@pytest.mark.parametrize("below", [10, 18, 22, 24.5, 27, 31])
+@pytest.mark.parametrize("d,dtype", [(64, torch.float16), (128, torch.float16), (128, torch.bfloat16)])
+def test_prefill_small_weights_beside_large_ones(device, below, d, dtype):
+    # a sink at the start of sequences whose tiles are cut and whole.  Beside the usual bound, float16's
+    # parts of a weight end 2^-38 below the largest (absolute error of each)
+    case = sink_case(840, [5000, 700, 300, 60], [40, 32, 90, 60], below, (0,), 8, 2, d, dtype)
+    ref, cond = PA.paged_attention(**oracle_args(case), terms=True)
+    if dtype == torch.float16:
+        places = PA.query_places(case["seq_lens"], case["query_start_loc"], case["query_lens"])
+        n = np.array([kv_len for _, kv_len, _ in places], dtype=np.float64)[:, None, None]
+        cond = cond + n * 2.0 ** -38 * 384 / (ARITH_K[dtype] * UNIT[dtype])   # 384: the values' largest
+    assert_close_to_oracle(run(case, device), (ref, cond), dtype)
