@@ -1707,6 +1707,28 @@ static int lm_check(const void* hidden, int64_t ld_hidden, const void* weight, i
   return NS_OK;
 }
 
+// Batch rows / 32 of a workgroup of the column-owner kernel (4, 6, 8 or 10; beyond 10 the accumulators and the
+// weight registers pass 256).  The fewest workgroup rows of up to 320 batch rows, equally tall to the next
+// multiple of 64, so that the products follow the batch and the weight is read once up to 320 rows; or
+// rows of 256 where those take fewer or cheaper rounds of the 256 CUs, one workgroup on each.  A round takes
+// time as 5/2 + TM (55, 66, 77 and 92 us at k = 2048 for TM = 4, 6, 8 and 10), one that fills the chip only
+// in part three quarters of that or 1/2 + 1/2 the part.  Taller rows or rows of 256, us:
+//   50257 x 4096: 300 rows 141 or 230, 600 rows 288 or 354, 1280 rows 568 or 547;
+//   32000 x 1024: 600 rows 58 or 77, 960 rows 101 or 94;
+//   16384 x 4096: 300 rows 114 or 95, 1100 rows 152 or 204.
+static int lm_cols_tiles(int32_t m, int32_t n) {
+  const int64_t groups = ((int64_t)m + 319) / 320;
+  const int64_t rows = ((int64_t)m + groups - 1) / groups;
+  const int tm = rows <= 128 ? 4 : 2 * (int)((rows + 63) / 64);
+  const int64_t gx = ((int64_t)n + ns::LM_NT - 1) / ns::LM_NT;
+  auto cost = [&](int t) -> int64_t {   // in 1/1024 of half a unit
+    const int64_t wgs = gx * (((int64_t)m + 32 * t - 1) / (32 * t)), part = wgs % 256;
+    const int64_t last = part == 0 ? 0 : part <= 128 ? 768 : 512 + 2 * part;
+    return (5 + 2 * t) * (wgs / 256 * 1024 + last);
+  };
+  return tm > 8 && cost(8) < cost(tm) ? 8 : tm;
+}
+
 static int lm_launch(const void* hidden, int64_t ld_hidden, int64_t n_hidden, const int64_t* rows, const void* weight,
                      int64_t ld_weight, void* logits, int64_t ld_logits, int32_t m, int32_t n, int32_t k, bool packed,
                      hipStream_t stream) {
@@ -1723,13 +1745,9 @@ static int lm_launch(const void* hidden, int64_t ld_hidden, int64_t n_hidden, co
   ns::LmParams P{static_cast<const uint16_t*>(hidden), ld_hidden, rows, n_hidden, static_cast<const uint16_t*>(weight),
                  packed ? 0 : ld_weight, static_cast<uint16_t*>(logits), ld_logits, m, n, k};
   // batches beyond 64 rows: the column-owner kernel (weight straight into registers); its hidden loads
-  // take 32-bit offsets.  Workgroup rows of up to 320 batch rows, the fewest that hold the batch and
-  // equally tall to the next multiple of 64, so that the products follow the batch and the weight is
-  // read once up to 320 rows (50257 x 4096 at 300 rows: 303 us with two workgroup rows of 256, 171 with one
-  // of 320; at 150 rows 115 with 256, 90 with 192)
+  // take 32-bit offsets
   if (packed && m > 64 && n_hidden * ld_hidden * 2 < (int64_t)0xffffffffu) {
-    const int64_t rows_wg = ((int64_t)m + ((int64_t)m + 319) / 320 - 1) / (((int64_t)m + 319) / 320);
-    const int tm = rows_wg <= 128 ? 4 : 2 * (int)((rows_wg + 63) / 64);
+    const int tm = lm_cols_tiles(m, n);
     const int64_t gyc = ((int64_t)m + 32 * tm - 1) / (32 * tm);
     if (gyc > 65535) return fail(NS_ERR_INVALID, "m too large");
     const dim3 gridc((unsigned)((n + ns::LM_NT - 1) / ns::LM_NT), (unsigned)gyc), blockc(ns::LM_THREADS);

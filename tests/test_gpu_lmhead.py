@@ -139,11 +139,13 @@ def test_packed_large_batch_gathers_rows_and_flags_bad_indices(device, m):
     assert torch.equal(out[good].contiguous().view(torch.int16), plain[good].contiguous().view(torch.int16))
 
 
-@pytest.mark.parametrize("m", [65, 128, 129, 192, 193, 257, 320, 321, 385, 641])
-def test_packed_batch_row_tiles(device, m):
+@pytest.mark.parametrize("m,vocab", [(65, 517), (128, 517), (129, 517), (192, 517), (193, 517), (257, 517), (320, 517),
+                                     (321, 517), (385, 517), (641, 517), (257, 31990), (320, 31990), (577, 31990),
+                                     (640, 31990), (960, 31990)])
+def test_packed_batch_row_tiles(device, m, vocab):
     """Every height of the column-owner kernel's workgroup rows (128, 192, 256, 320) at its edges, one
-    to three of them: the same bits as the weight as stored."""
-    hidden, weight = make(device, m, 517, 256, seed=57 + m, scale=2.0)
+    to four of them: the same bits as the weight as stored."""
+    hidden, weight = make(device, m, vocab, 256, seed=57 + m, scale=2.0)
     packed = L.lm_head_bf16(hidden, L.PackedLmHead(weight))
     plain = L.lm_head_bf16(hidden, weight)
     torch.cuda.synchronize()
