@@ -111,26 +111,29 @@ def test_lm_head_special_values(device):
     assert bool(((ours[fin] - ref[fin]).abs() <= ref[fin].abs() * 2.0 ** -8 + 1e-3).all())
 
 
-@pytest.mark.parametrize("m", [100, 260])
-def test_packed_large_batch_gathers_rows_and_flags_bad_indices(device, m):
-    """Packed batches beyond 64 rows (the column-owner kernel, one and two workgroup rows):
-    gathered rows, a padded hidden stride, invalid indices as NaN rows, a logits buffer wider
-    than the vocab; the same bits as the weight as stored."""
-    hidden_full, weight = make(device, 700, 1300, 192, seed=31 + m, scale=3.0)
+@pytest.mark.parametrize("m,vocab", [(100, 1300), (260, 1300), (150, 1300), (260, 31990), (330, 1300), (600, 31990),
+                                     (641, 1300)])
+def test_packed_large_batch_gathers_rows_and_flags_bad_indices(device, m, vocab):
+    """Packed batches beyond 64 rows (the column-owner kernel at each height of its workgroup rows: one of
+    128, two of 256, one of 192, one of 320, two of 192, two of 320 and three of 256 batch rows): gathered
+    rows, a padded hidden stride, invalid indices as NaN rows at the edges of workgroup rows and tiles, a
+    logits buffer wider than the vocab; the same bits as the weight as stored."""
+    hidden_full, weight = make(device, 700, vocab, 192, seed=31 + m, scale=3.0)
     hidden = torch.zeros((700, 200), dtype=torch.bfloat16, device=device)[:, :192]
     hidden.copy_(hidden_full)
     g = np.random.default_rng(m)
     rows_np = g.integers(0, 700, size=m).astype(np.int64)
-    bad_pos = g.choice(m, 5, replace=False)
-    rows_np[bad_pos] = np.array([-1, 700, 701, -5, 1 << 40], dtype=np.int64)
+    edges = {0, 31, 32, 63, 64, 127, 128, 191, 192, 255, 256, 319, 320, 383, 384, 511, 512, 575, 576, m - 1}
+    bad_pos = np.array(sorted({e for e in edges if e < m} | {int(x) for x in g.choice(m, 5, replace=False)}))
+    rows_np[bad_pos] = np.resize(np.array([-1, 700, 701, -5, 1 << 40], dtype=np.int64), bad_pos.size)
     rows = torch.from_numpy(rows_np).to(device)
     pw = L.PackedLmHead(weight)
-    out_full = torch.full((m, 1400), 7.0, dtype=torch.bfloat16, device=device)
-    out = out_full[:, :1300]
+    out_full = torch.full((m, vocab + 100), 7.0, dtype=torch.bfloat16, device=device)
+    out = out_full[:, :vocab]
     L.lm_head_bf16(hidden, pw, rows=rows, out=out)
     plain = L.lm_head_bf16(hidden, weight, rows=rows)
     torch.cuda.synchronize()
-    assert bool((out_full[:, 1300:] == 7.0).all())   # nothing written past n
+    assert bool((out_full[:, vocab:] == 7.0).all())   # nothing written past n
     bad = torch.zeros(m, dtype=torch.bool, device=device)
     bad[torch.from_numpy(bad_pos).to(device)] = True
     assert bool(torch.isnan(out.float()[bad]).all())
