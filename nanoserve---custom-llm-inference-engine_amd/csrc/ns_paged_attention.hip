@@ -1103,7 +1103,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
   __shared__ int s_bad;        // an invalid block met in this segment
   __shared__ int s_last;
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, c32 = lane & 31;
+  const int wave = threadIdx.x >> 6;
   const int n_tiles = f.n_tiles;
 
   // The workgroup's units: unit u of all hkv * S steps is step u % S of the tiles in order, KV
@@ -1113,6 +1113,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
   int64_t u0 = 0, u1 = 0, per = 1, S = 0;
   int w = 0, tile = 0, off = 0, kvh = 0;
   if (f.grid > 0) {
+    const int tid = threadIdx.x, lane = tid & 63;
     const int q = (n_tiles + kPfThreads - 1) / kPfThreads;   // tiles per thread, consecutive
     const int first = tid * q;
     int64_t mine = 0;
@@ -1165,7 +1166,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     tile = blockIdx.x % n_tiles;
     kvh = blockIdx.x / n_tiles;
     const PfTile t = pf_tile(p, f, tile, BQ);
-    if (tid == 0 && kvh == 0 && p.status) {
+    if (threadIdx.x == 0 && kvh == 0 && p.status) {
       if (t.steps == 0) atomicOr(p.status, NS_PA_STATUS_BAD_TILE);
       if (t.cut) atomicOr(p.status, NS_PA_STATUS_SEQ_TOO_LONG);
     }
@@ -1173,24 +1174,11 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     u1 = t.steps;
   }
 
-  // every chunk of the thread has dims 8 dc .. + 7 (kPfThreads is a multiple of CPP); the host
-  // keeps token strides times block_size below 2^31, so a slot's offset is a 32-bit product
-  const int dc0 = tid % CPP;
+  // the host keeps token strides times block_size below 2^31, so a slot's offset is a 32-bit product
   const int sk_tok = (int)p.sk_tok, sv_tok = (int)p.sv_tok;
   constexpr int PW = 64 / CPP;   // positions of a wave's load instruction
   const int wv = __builtin_amdgcn_readfirstlane(wave);
-  const uint32_t koff = (uint32_t)(lane / CPP * sk_tok) * 2u + 16u * dc0;
-  const uint32_t voff = (uint32_t)(lane / CPP * sv_tok) * 2u + 16u * dc0;
-  // The transposing read (ds_read_b64_tr_b16): in each 16-lane group, lane j's four results are
-  // element j % 4 of the 4-element rows that lanes 4 m + j / 4 address, m = 0..3.  So that lane L
-  // receives positions 16 s + 4 h + m of dim 32 db + L % 32, lane L addresses position
-  // 16 s + 4 (L / 32) + (L % 16) / 4, dims 32 db + 16 ((L / 16) % 2) + 4 (L % 4) .. + 3.
-  const int tr_pos = 4 * (lane >> 5) + ((lane & 15) >> 2);
-  const int tr_dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
   const float scale = f.scale_log2;
-  // the lane's column: token tok, head hd
-  const int c = wave * 32 + c32;
-  const int tok = c / G, hd = c % G;
 
   for (int64_t u = u0; u < u1;) {
     if (tile == n_tiles) {
@@ -1202,6 +1190,29 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
       ++tile;
       continue;
     }
+    // The lane's places and offsets.  At 128 dims they are made anew for each tile, from the lane's number (the
+    // empty asm hides that it is the same each time): kept across the merge of a cut tile, whose loads in
+    // flight take 64 registers, 11 to 15 of them spilled to scratch memory.
+    int tid = threadIdx.x;
+    if constexpr (D == 128) {
+      uint32_t lanes = 0xffffffffu;
+      asm volatile("" : "+s"(lanes));
+      tid = 64 * wv + __builtin_amdgcn_mbcnt_hi(lanes, __builtin_amdgcn_mbcnt_lo(lanes, 0u));
+    }
+    const int lane = tid & 63, h = lane >> 5, c32 = lane & 31;
+    // every chunk of the thread has dims 8 dc0 .. + 7 (kPfThreads is a multiple of CPP)
+    const int dc0 = tid % CPP;
+    const uint32_t koff = (uint32_t)(lane / CPP * sk_tok) * 2u + 16u * dc0;
+    const uint32_t voff = (uint32_t)(lane / CPP * sv_tok) * 2u + 16u * dc0;
+    // The transposing read (ds_read_b64_tr_b16): in each 16-lane group, lane j's four results are
+    // element j % 4 of the 4-element rows that lanes 4 m + j / 4 address, m = 0..3.  So that lane L
+    // receives positions 16 s + 4 h + m of dim 32 db + L % 32, lane L addresses position
+    // 16 s + 4 (L / 32) + (L % 16) / 4, dims 32 db + 16 ((L / 16) % 2) + 4 (L % 4) .. + 3.
+    const int tr_pos = 4 * (lane >> 5) + ((lane & 15) >> 2);
+    const int tr_dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    // the lane's column: token tok, head hd
+    const int c = wv * 32 + c32;
+    const int tok = c / G, hd = c % G;
     const int take = (int)(u1 - u < t.steps - off ? u1 - u : t.steps - off);
     // visible positions of the lane's column (-1: a padding column, never written)
     int kvl = -1;
@@ -1457,7 +1468,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
       constexpr int SW = D / 2 * 64;   // floats of a slot per wave
       const int mine = w == wa ? begin_slot : w;
       if (live) {
-        float* dst = f.ws_acc + ((int64_t)mine * kPfWaves + wave) * SW + 2 * lane;
+        float* dst = f.ws_acc + ((int64_t)mine * kPfWaves + wv) * SW + 2 * lane;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -1484,8 +1495,8 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
           for (int i = wa; i <= wb; ++i) {
-            const int64_t slot = i == wa ? begin_slot : i;
-            const float* src = f.ws_acc + (slot * kPfWaves + wave) * SW + 2 * lane;
+            const int64_t slot = __builtin_amdgcn_readfirstlane(i == wa ? begin_slot : i);
+            const float* src = f.ws_acc + (slot * kPfWaves + wv) * SW + 2 * lane;
             const f32x2 ml = ld_dev2(f.ws_ml + (slot * kPfCols + c) * 2);
             f32x2 a[D / 4];   // all of a segment's loads issued before the first is used
 #pragma unroll

@@ -128,3 +128,20 @@ def test_argument_errors_without_a_gpu():
     # an empty batch is a no-op
     a.total_q = 0
     assert lib.ns_paged_attention(ctypes.byref(a), None) == 0
+
+
+def test_no_kernel_uses_scratch(tmp_path):
+    """Every kernel of the library as built keeps its values in registers (a private segment slows each
+    dispatch): the sizes recorded in the code object's metadata."""
+    built()
+    llvm = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin")
+    fat, code = str(tmp_path / "fat"), str(tmp_path / "code")
+    subprocess.run([f"{llvm}/llvm-objcopy", "--dump-section", f".hip_fatbin={fat}", PA.LIB_PATH, str(tmp_path / "copy")],
+                   check=True)
+    subprocess.run([f"{llvm}/clang-offload-bundler", "--unbundle", "--type=o", f"--input={fat}", f"--output={code}",
+                    "--targets=hipv4-amdgcn-amd-amdhsa--gfx950"], check=True)
+    notes = subprocess.run([f"{llvm}/llvm-readelf", "--notes", code], check=True, capture_output=True, text=True).stdout
+    sizes = re.findall(r"\.private_segment_fixed_size:\s*(\d+)", notes)
+    names = re.findall(r"\.symbol:\s*(\S+)", notes)
+    assert len(sizes) == len(names) > 0
+    assert [n for n, size in zip(names, sizes) if int(size)] == []
