@@ -89,41 +89,15 @@ template <> struct Elem<float> { static constexpr int bytes = 4; };
 template <> struct Elem<Bf16> { static constexpr int bytes = 2; };
 template <> struct Elem<F16> { static constexpr int bytes = 2; };
 
-// N consecutive elements (N * bytes a multiple of 16, 16-byte aligned) as raw 16-byte words ...
-template <typename T, int N>
-struct Raw {
-  static constexpr int kVec = N * Elem<T>::bytes / 16;
-  u32x4 w[kVec];
-};
-
-template <typename T, int N>
-__device__ __forceinline__ void load_raw(const void* base, int64_t elem_off, Raw<T, N>& r) {
-  const u32x4* p = reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(base) + elem_off * Elem<T>::bytes);
+// N consecutive floats (N a multiple of 4, 16-byte aligned)
+template <int N>
+__device__ __forceinline__ void load_floats(const void* base, int64_t elem_off, float (&x)[N]) {
+  const u32x4* p = reinterpret_cast<const u32x4*>(reinterpret_cast<const float*>(base) + elem_off);
 #pragma unroll
-  for (int i = 0; i < Raw<T, N>::kVec; ++i) r.w[i] = p[i];
-}
-
-// ... converted to float
-template <typename T, int N>
-__device__ __forceinline__ void to_float(const Raw<T, N>& r, float (&x)[N]) {
-  const uint32_t* u = reinterpret_cast<const uint32_t*>(r.w);
-  if constexpr (Elem<T>::bytes == 4) {
+  for (int i = 0; i < N / 4; ++i) {
+    const u32x4 w = p[i];
 #pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = __uint_as_float(u[i]);
-  } else if constexpr (__is_same(T, Bf16)) {
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-      x[2 * i] = __uint_as_float(u[i] << 16);
-      x[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-      const _Float16 lo = __builtin_bit_cast(_Float16, (uint16_t)(u[i] & 0xFFFFu));
-      const _Float16 hi = __builtin_bit_cast(_Float16, (uint16_t)(u[i] >> 16));
-      x[2 * i] = (float)lo;
-      x[2 * i + 1] = (float)hi;
-    }
+    for (int j = 0; j < 4; ++j) x[4 * i + j] = __uint_as_float(w[j]);
   }
 }
 
@@ -408,7 +382,8 @@ __device__ __forceinline__ void finish_partition(const PaParams& p, int qi, int 
   }
 }
 
-template <typename T, int D, int G>
+// float32: vector arithmetic, a partition's scores in LDS.
+template <int D, int G>
 __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   // L lanes per KV position, DS dims each: 8 lanes, or 16 for eight heads of 128 dims (the query
   // slices and accumulators of eight heads would not fit the registers at 16 dims a lane)
@@ -440,7 +415,7 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   if (part >= n_parts) {
     if (part == 0) {  // no visible key: zeros (the reference's l == 0 guard, :103-104)
       for (int i = threadIdx.x; i < G * D; i += kThreads)
-        store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)(kvh * G + i / D) * p.so_head + i % D, 0.f);
+        store_one<float>(p.out, (int64_t)qi * p.so_tok + (int64_t)(kvh * G + i / D) * p.so_head + i % D, 0.f);
     }
     return;
   }
@@ -466,9 +441,7 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   float qv[G][DS];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    Raw<T, DS> r;
-    load_raw<T, DS>(p.q, (int64_t)qi * p.sq_tok + (int64_t)(kvh * G + g) * p.sq_head + dl * DS, r);
-    to_float<T, DS>(r, qv[g]);
+    load_floats(p.q, (int64_t)qi * p.sq_tok + (int64_t)(kvh * G + g) * p.sq_head + dl * DS, qv[g]);
 #pragma unroll
     for (int i = 0; i < DS; ++i) qv[g][i] *= p.scale_log2;
   }
@@ -493,26 +466,24 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   // pass 1: scores -> LDS. A wave takes batches of kBatch positions (wave w: batches w, w + 4, ...);
   // each lane requests its kSub rows of the batch before any arithmetic.
   for (int base = wave * kBatch; base < n; base += kWaves * kBatch) {
-    Raw<T, DS> raw[kSub];
+    float kx[kSub][DS];
     int blk[kSub];
 #pragma unroll
     for (int r = 0; r < kSub; ++r) {
       int off = 0;
       blk[r] = block_of(base + r * NSLOT + slot, off);
       if (blk[r] >= 0)
-        load_raw<T, DS>(p.k, (int64_t)blk[r] * p.sk_blk + (int64_t)off * p.sk_tok + (int64_t)kvh * p.sk_head + dl * DS,
-                        raw[r]);
+        load_floats(p.k, (int64_t)blk[r] * p.sk_blk + (int64_t)off * p.sk_tok + (int64_t)kvh * p.sk_head + dl * DS,
+                    kx[r]);
     }
 #pragma unroll
     for (int r = 0; r < kSub; ++r) {
-      float kx[DS];
-      to_float<T, DS>(raw[r], kx);
       const int j = base + r * NSLOT + slot;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         float sc = 0.f;
 #pragma unroll
-        for (int i = 0; i < DS; ++i) sc = fmaf(qv[g][i], kx[i], sc);
+        for (int i = 0; i < DS; ++i) sc = fmaf(qv[g][i], kx[r][i], sc);
         sc = L == 8 ? octet_sum(sc) : hex_sum(sc);
         if (dl == g && j < n) s_score[g * kMaxPart + j] = blk[r] >= 0 ? sc : -INFINITY;
       }
@@ -520,7 +491,7 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   }
   // the wave's first value batch is requested before the softmax pass: the workgroups of a CU
   // reach that pass together, and the requests keep the memory pipe busy across it
-  Raw<T, DS> vraw[kSub];
+  float vx[kSub][DS];
   int vblk[kSub];
   auto request_values = [&](int base) {
 #pragma unroll
@@ -528,8 +499,8 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
       int off = 0;
       vblk[r] = block_of(base + r * NSLOT + slot, off);
       if (vblk[r] >= 0)
-        load_raw<T, DS>(p.v, (int64_t)vblk[r] * p.sv_blk + (int64_t)off * p.sv_tok + (int64_t)kvh * p.sv_head + dl * DS,
-                        vraw[r]);
+        load_floats(p.v, (int64_t)vblk[r] * p.sv_blk + (int64_t)off * p.sv_tok + (int64_t)kvh * p.sv_head + dl * DS,
+                    vx[r]);
     }
   };
   request_values(wave * kBatch);
@@ -565,14 +536,12 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
 #pragma unroll
     for (int r = 0; r < kSub; ++r) {
       if (vblk[r] < 0) continue;
-      float vx[DS];
-      to_float<T, DS>(vraw[r], vx);
       const int j = base + r * NSLOT + slot;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         const float w = s_score[g * kMaxPart + j];
 #pragma unroll
-        for (int i = 0; i < DS; ++i) acc[g][i] = fmaf(w, vx[i], acc[g][i]);
+        for (int i = 0; i < DS; ++i) acc[g][i] = fmaf(w, vx[r][i], acc[g][i]);
       }
     }
   }
@@ -589,7 +558,7 @@ __global__ __launch_bounds__(kThreads) void pa_partition_kernel(PaParams p) {
   }
   __syncthreads();
 
-  finish_partition<T, D, G>(p, qi, kvh, part, n_parts,
+  finish_partition<float, D, G>(p, qi, kvh, part, n_parts,
                             [&](int w, int g, int d) { return s_red[(w * G + g) * D + d]; }, s_m, s_l, s_score,
                             nullptr, []() {});
 }
@@ -1596,26 +1565,21 @@ uint64_t workspace_bytes(int32_t total_q, int32_t hq, int32_t hkv, int32_t head_
 // when f.tiles is set (16-bit types only)
 template <typename T, int D, int G>
 void launch(const PaParams& p, const PfParams& f, int n_tokens, int n_tiles, hipStream_t stream) {
-  // scalar row addresses: power-of-two blocks that hold a wave's load, block strides in 32 bits
-  const bool by_wave = p.bs_shift >= 0 && p.block_size >= 512 / D && p.sk_blk >= 0 && p.sv_blk >= 0 &&
-                       p.sk_blk < INT32_MAX && p.sv_blk < INT32_MAX;
-  (void)by_wave;
-  if (n_tokens > 0) {
-    dim3 grid(n_tokens, p.hkv, p.max_parts > 0 ? p.max_parts : 1);
-    if constexpr (Elem<T>::bytes == 2) {
+  const dim3 grid(n_tokens, p.hkv, p.max_parts > 0 ? p.max_parts : 1);
+  if constexpr (Elem<T>::bytes == 4) {
+    if (n_tokens > 0) hipLaunchKernelGGL((pa_partition_kernel<D, G>), grid, dim3(kThreads), 0, stream, p);
+  } else {
+    // scalar row addresses: power-of-two blocks that hold a wave's load, block strides in 32 bits
+    const bool by_wave = p.bs_shift >= 0 && p.block_size >= 512 / D && p.sk_blk >= 0 && p.sv_blk >= 0 &&
+                         p.sk_blk < INT32_MAX && p.sv_blk < INT32_MAX;
+    const dim3 tiles((unsigned)(f.grid > 0 ? f.grid : n_tiles * p.hkv));
+    if (n_tokens > 0) {
       if (by_wave) hipLaunchKernelGGL((pa_decode_kernel<T, D, G, true>), grid, dim3(kThreads), 0, stream, p);
       else hipLaunchKernelGGL((pa_decode_kernel<T, D, G, false>), grid, dim3(kThreads), 0, stream, p);
-    } else {
-      hipLaunchKernelGGL((pa_partition_kernel<T, D, G>), grid, dim3(kThreads), 0, stream, p);
     }
-  }
-  if constexpr (Elem<T>::bytes == 2) {
     if (n_tiles > 0) {
-      const dim3 grid((unsigned)(f.grid > 0 ? f.grid : n_tiles * p.hkv));
-      if (by_wave)
-        hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, true>), grid, dim3(kPfThreads), 0, stream, p, f);
-      else
-        hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, false>), grid, dim3(kPfThreads), 0, stream, p, f);
+      if (by_wave) hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, true>), tiles, dim3(kPfThreads), 0, stream, p, f);
+      else hipLaunchKernelGGL((pa_prefill_kernel<T, D, G, false>), tiles, dim3(kPfThreads), 0, stream, p, f);
     }
   }
 }
