@@ -13,7 +13,12 @@
  * 0 .. min(kv_pos, seq_lens[s]-1) of its sequence; KV position t lives in physical block
  * block_tables[s][t / block_size], slot t % block_size. Query head h reads KV head
  * h / (num_heads_q / num_kv_heads) (GQA). out = softmax(scale * q.K^T) V in float32 arithmetic,
- * rounded to the query's dtype; a query with no visible key gets zeros.
+ * rounded to the query's dtype; a query with no visible key gets zeros.  For bfloat16 and float16 the
+ * scores, their sums and the accumulators are float32, and a softmax weight w (relative to its
+ * column's largest) enters the value product as two 16-bit parts: to 2^-17 w in bfloat16, to 2^-22 w
+ * + 2^-49 (prefill tiles: 2^-38) in float16.  An infinite value in a visible row gives infinity, except
+ * in a prefill tile, whose outputs are NaN in that dim for the tokens that see it and for those
+ * up to 63 positions before it.
  *
  * Layouts: query/out (total_q, num_heads_q, head_dim), caches (num_blocks, block_size,
  * num_kv_heads, head_dim), each with arbitrary element strides except a unit head_dim stride and
@@ -114,11 +119,11 @@ int ns_paged_attention_workspace_bytes(int32_t total_q, int32_t num_heads_q, int
  * n_prefill_tiles * num_kv_heads for the tiles; zero-filled once, left zeroed by every call. */
 int ns_paged_attention_call_workspace(const ns_paged_attn_args* args, uint64_t* bytes, uint64_t* counters);
 
-/* Paged attention (paged_attention_triton.py:134-170, paged_attention_torch.py:31-100): one
- * launch; one workgroup per (query token, KV head, KV partition) computes all query heads of that
- * KV head, so each key and value row is read once per query token; when a query spans several
- * partitions the last of them to finish merges them. Returns 0 on success, nonzero on invalid
- * arguments. */
+/* Paged attention (paged_attention_triton.py:134-170, paged_attention_torch.py:31-100): one launch
+ * for the per-token queries, one for the prefill tiles. A per-token workgroup (query token, KV head,
+ * KV partition) computes all query heads of that KV head, so each key and value row is read once
+ * per query token; when a query spans several partitions the last of them to finish merges them.
+ * Returns 0 on success, nonzero on invalid arguments. */
 int ns_paged_attention(const ns_paged_attn_args* args, hipStream_t stream);
 
 #ifdef __cplusplus

@@ -9,17 +9,19 @@
 //    that KV head (G = num_heads_q / num_kv_heads of them), so each key and value row is read from
 //    HBM once per query token instead of once per query head as the reference's per-(token, head)
 //    programs do.  The 16-bit types take pa_decode_kernel (matrix core), float32 pa_partition_kernel
-//    (vector arithmetic; the two points below are its).
-//  * Lane layout per wave step: 16 KV positions, 8 lanes per position, each lane holding a
-//    head_dim/8 slice (32 contiguous bytes of a bf16 row at head_dim 128: two 16-byte loads). The
-//    slice's partial dot products are summed across the 8 lanes with ds_swizzle (no LDS traffic).
+//    (vector arithmetic; the next two points are its).
+//  * Lane layout per wave batch: 16 KV positions, 8 at a time, 8 lanes per position, each lane holding a
+//    head_dim/8 slice (64 contiguous bytes at head_dim 128: four 16-byte loads; G = 8 at head_dim 128:
+//    8 positions, 16 lanes each, 32 bytes a lane).  The slice's partial dot products are summed across
+//    the position's lanes with ds_swizzle (no LDS traffic).
 //  * Exact two-pass softmax inside a partition: scores (already in log2 units) go to LDS, one max
-//    and one exp2 pass over LDS, then the value pass. Partitions of a long sequence (split-KV,
-//    sized on the host so that the grid holds >= 1024 workgroups) are merged by the last of the
-//    row's workgroups to arrive (max-rescaled sums); a query that fits one partition is written
-//    directly. One launch per call.
-//  * The sequence of a query token and its KV position are computed in the kernel (binary search
-//    over query_start_loc), so a call needs no host copy of the batch layout.
+//    and one exp2 pass over LDS, then the value pass.
+//  * Partitions of a long sequence (split-KV, sized on the host so that the grid holds >= 1024
+//    workgroups) are merged by the last of the row's workgroups to arrive (max-rescaled sums); a
+//    query that fits one partition is written directly.  One launch for the decode tokens of a call,
+//    one for its prefill tiles.
+//  * The sequence of a query token and its KV position are computed in the kernel (a search over
+//    query_start_loc, 64 entries at a time), so a call needs no host copy of the batch layout.
 
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -34,14 +36,15 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kSub = 2;                 // KV positions per lane per batch
-constexpr int kMaxPart = 1024;          // largest KV partition (LDS score buffer)
+constexpr int kMaxPart = 1024;          // largest KV partition (LDS score buffer, block list)
 constexpr int kMinPart = 64;
 // partitions of a row merged through a table of their weights in LDS (one long row of few KV heads has
 // hundreds): the loop that takes more reads three words per partition and output one after the other.
 // one row of 17000 .. 65536 positions, 1 .. 3 KV heads (266 .. 1024 partitions, bf16, head_dim 128,
 // G = 1 .. 8): 29-296 us with the table, 75-1145 by the loop
 constexpr int kMaxMerge = 1024;
-constexpr int kTargetGroups = 1024;     // workgroups a launch aims for before splitting stops
+// workgroups a launch aims for before splitting stops: four per CU (the 128-dim 16-bit kernels hold three at once)
+constexpr int kTargetGroups = 1024;
 constexpr float kLog2e = 1.4426950408889634f;
 
 thread_local char g_err[512];
@@ -645,25 +648,27 @@ __device__ __forceinline__ void plain_partition(const PaParams& p, int qi, int k
 // vector unit did about 165 instructions per 8 positions at G = 3 (the dot products, their lane sums,
 // the widening) and the passes of all the workgroups of a launch fell together, so that the memory
 // pipe idled across the softmax.
-//   * A wave takes steps of 32 positions.  A load instruction of
-//     a wave covers whole rows (4 of 128 dims, 8 of 64), so that every 128-byte line is taken at one
-//     touch: loading the products' operand layout (16 rows by 64 bytes) directly, with 128 KB in flight
-//     on a CU, evicted lines between their touches (64 x 2048 at G = 3: 114 us, and 105 at half the
-//     waves).  A step's loads are issued before the previous step's arithmetic (8 KB a wave in flight)
-//     and go through the wave's own LDS rows.
+//   * A wave takes steps of 16 positions at 128 dims, 32 at 64 (8 KB of rows either way).  A load
+//     instruction of a wave covers whole rows (4 of 128 dims, 8 of 64), so that every 128-byte line is
+//     taken at one touch: loading the products' operand layout (16 rows by 64 bytes) directly was
+//     slower with 128 KB in flight on a CU (64 x 2048 at G = 3: 114 us) than with half of it (105), as if
+//     lines left the cache between their touches.  A step's loads are issued before the previous
+//     step's arithmetic (8 KB a wave in flight) and go through the wave's own LDS rows.
 //   * S^T: lane l holds head l % 16 at positions 16 b + 4 (l / 16) + i of row block b.  Its weights are
-//     the B operand of O^T += V^T P^T as they are, with k-slot i of quarter l / 16 at position
-//     4 (l / 16) + i for i < 4, else 12 + 4 (l / 16) + i; the V^T operand is read in that order by two
-//     transposing reads from the wave's own LDS rows.  P goes in as a high and a low 16-bit part (Mma);
+//     the B operand of O^T += V^T P^T as they are: a 16x16x16 product per 16 dims at 128 dims, k-slot i
+//     of quarter l / 16 at position 4 (l / 16) + i; a 16x16x32 one at 64, whose k-slots 4 .. 7 are the
+//     second row block's.  The V^T operand is read in that order by one transposing read (two at 64
+//     dims) from the wave's own LDS rows.  P goes in as a high and a low 16-bit part (Mma);
 //     float16's low parts are summed apart and scaled back (64 rows of up to 2048, 128 dims: 60.3 us
 //     without, 61.5 with).
 //   * LDS rows are unpadded; 16-byte chunk c of row r sits at c ^ swz(r), under which the 16 rows of a
 //     write and the 8 rows of a transposing read hit the 64 banks once.
 // Bound by HBM.  Measured (bf16, 8 KV heads of 128 dims, blocks of 16; the vector form, then this):
-// 8 x 8192 at G = 3: 61 -> 58 us; 64 x 2048: 107 -> 107 (5.0 TB/s); 256 rows of up to 512: 77 -> 57;
-// G = 4, 64 rows of up to 2048: 130 -> 80; G = 8, 32 rows of up to 2048: 134 -> 37.  At 128 dims three
-// waves a SIMD (168 registers): four spill 8 bytes and measured 63, 111 and 63 us on the first three,
-// two 61, 103 and 60.
+// 8 x 8192 at G = 3: 60 -> 58 us; 64 x 2048: 108 -> 108 (5.0 TB/s); 256 x 512: 107 -> 98; G = 4, 64 x 2048:
+// 141 -> 108; G = 8, 64 x 2048: 310 -> 113.  G = 1 gains least: one row of 64 to 8 of 300 positions 5-12%
+// faster, 8 x 2048 20.2 -> 20.9, 64 x 2048 of 64 dims 47 -> 50.  At 128 dims three waves a SIMD (138 to 150
+// registers of 168): four spill 8 bytes and measured 63 us at 8 x 8192, 111 at 64 x 2048 and 63 at 256 rows
+// of up to 512, two 61, 103 and 60, three 58, 107 and 57.
 // BW as in the prefill kernel: a row's address is a scalar plus a lane's fixed offset.
 template <typename T, int D, int G, bool BW>
 __global__ __launch_bounds__(kThreads)
@@ -842,7 +847,7 @@ __global__ __launch_bounds__(kThreads)
       }
     }
 
-    // online softmax of head c16 over the step's 32 positions, 8 of them in this lane
+    // online softmax of head c16 over the step's positions, 4 NB of them in this lane
     float mt = -INFINITY;
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -946,14 +951,13 @@ __global__ __launch_bounds__(kThreads)
 
 // ---- prefill kernel: query tiles on MFMA -------------------------------------------------------
 //
-// Sequences with several query tokens (chunked prefill) go by query tile: one workgroup of four
-// waves per (tile, KV head, KV partition) holds kPfCols = 128 query columns -- kPfCols / G tokens
-// of one sequence times the G query heads of the KV head, column c = token (c / G), head (c % G),
-// 32 columns per wave -- and walks the partition's positions 64 at a time.  Each step's key and
-// value rows are read from memory once for the whole tile (all 256 threads load them into LDS:
-// keys as rows, values transposed, dims as rows), so each row is read once per 128 columns
-// instead of once per query token.  On v_mfma_f32_32x32x16 (bf16 or f16 operands, float32
-// accumulation), per wave:
+// Sequences with several query tokens (chunked prefill) go by query tile: kPfCols = 128 query columns
+// -- kPfCols / G tokens of one sequence times the G query heads of a KV head, column c = token
+// (c / G), head (c % G) -- taken by a workgroup of four waves, 32 columns each, which walks a run of
+// the sequence's positions 64 at a time.  Each step's key and value rows are read from memory once
+// for the whole tile (all 256 threads load them into LDS, as rows), so each row is read once per
+// 128 columns instead of once per query token.  On v_mfma_f32_32x32x16 (bf16 or f16 operands,
+// float32 accumulation), per wave:
 //   * S^T = K Q^T for the step's two 32-position row blocks: rows positions, columns the wave's
 //     queries.  A lane holds one query column (lane % 32) of 16 positions per block, so the
 //     online softmax of a column (max, exp2, sum) runs in the lane plus one exchange with
@@ -961,23 +965,24 @@ __global__ __launch_bounds__(kThreads)
 //   * O^T += V^T P^T over the step's four 16-position k-steps, the probabilities taken straight
 //     from the S^T layout as the B operand: k-slot i of the lanes of half h is position
 //     16 s + 8 (i / 4) + 4 h + i % 4 of the step, and the V^T operand is read in that order from
-//     the transposed value rows (two 8-byte reads).  P goes in as two 16-bit parts, hi = RN(p)
+//     the value rows by two transposing LDS reads.  P goes in as two 16-bit parts, hi = RN(p)
 //     and lo = RN(p - hi), whose products with a value are exact in float32: bfloat16 carries p to
 //     about 2^-17 relative, float16 to 2^-22 and 2^-38 of the column's largest weight (Mma; its low
 //     parts summed apart, as in the decode kernel, took 5 to 9% more), where a single 16-bit P
-//     would round each weight by up to 2^-9.
+//     would round each weight by up to 2^-9.  The parts of a weight times an infinite value are
+//     NaN, also for a position of the step that the causal cut hides from the column.
 // The scores are the float32 dot products times scale * log2(e) (folded into the exponent's fma)
 // and exp2 replaces exp, as in the decode kernel.
 //
 // Work split: all steps of all (tile, KV head) pairs are shared evenly by up to 512 workgroups (two
 // per CU, all resident), each taking a run of consecutive steps, so that they end together whatever
 // the sequences' lengths and a tile is cut only where a run ends: at most two partials per
-// workgroup, stored and merged in the lanes' accumulator layout (256 contiguous bytes per 4-byte
-// element of a wave).  Four 512-token chunks ending at 2048 .. 8192 positions (24 / 8 heads of 128
-// dims, bf16): 627 -> 257 us, 195 -> 475 TFLOP/s (223 us, 545 TFLOP/s with scalar row addresses),
-// against partitions of at most 1024 positions whose
-// 64 KB of partials each went out and came back as scattered 4-byte accesses; three chunks of up to
-// 417 tokens beside 29 decode rows (32 / 8 heads of 64 dims, f16): 89 -> 55 us for the call.
+// workgroup, stored and merged in the lanes' accumulator layout (8 bytes a lane, 512 contiguous bytes a
+// store).  Four 512-token chunks ending at 2048 .. 8192 positions (24 / 8 heads of 128 dims, bf16): 627 ->
+// 257 us, 195 -> 475 TFLOP/s, against partitions of at most 1024 positions whose 64 KB of partials
+// each went out and came back as scattered 4-byte accesses; 228 us, 535 TFLOP/s with scalar row
+// addresses; three chunks of up to 417 tokens beside 29 decode rows (32 / 8 heads of 64 dims, f16):
+// 89 -> 55 us for the call.
 // Keys and values are double buffered in LDS (one barrier a step), the value rows at a pitch under
 // which a transposing read's four rows hit different banks (the key rows' pitch left them 4-way
 // conflicted), and the block table is read one step ahead of the rows instead of through LDS.
@@ -1049,7 +1054,7 @@ __device__ __forceinline__ f32x2 ld_dev2(const float* p) {
 // BW: the block size is a power of two and at least the consecutive positions one load instruction
 // of a wave covers (4 at 128 dims, 8 at 64), so these never straddle two blocks: the block is the
 // wave's, and a row's address a scalar address plus a lane's fixed offset instead of 64-bit products
-// per lane (four 512-token chunks up to 8192 positions: 252 -> 223 us).
+// per lane (four 512-token chunks up to 8192 positions: 257 -> 228 us).
 template <typename T, int D, int G, bool BW>
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void pa_prefill_kernel(PaParams p,
                                                                                                         PfParams f) {
@@ -1505,7 +1510,10 @@ int pf_part_tokens_for(int32_t n_tiles, int32_t hkv, int32_t max_seq_len) {
 // tiles are cut when the longest could be (max_seq_len above the partition length above, which
 // shrinks while there are fewer than 512 of them).  512 workgroups are all resident at once, so
 // equal shares end together.  Fewer, so that the slots they need stay within the partials' room
-// of one slot per (tile, KV head, partition).
+// of one slot per (tile, KV head, partition).  With few tiles that costs nothing throughout: one tile of
+// 16 tokens, 24 / 8 heads of 128 dims, with this grid, and with one workgroup per (tile, KV head,
+// partition) and the room it needs: 300 positions 18.0 and 22.7 us, 512 24.2 and 19.4, 600 21.5 and
+// 23.8, 700 28.2 and 24.9, 1100 28.1 and 25.7 (a workgroup per partition of 256, before: 30.7 to 40.7).
 int pf_grid_for(int32_t n_tiles, int32_t hkv, int32_t max_seq_len) {
   if (n_tiles <= 0) return 0;
   const int part = pf_part_tokens_for(n_tiles, hkv, max_seq_len);

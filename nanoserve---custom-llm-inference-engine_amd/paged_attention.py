@@ -16,7 +16,7 @@ Differences from the reference's launcher, all on the host side:
     host once, as the reference's launcher reads ``seq_lens.tolist()`` and ``query_lens.tolist()``
     (paged_attention_triton.py:120-121, paged_attention_torch.py:51): sequences of at least
     ``PREFILL_MIN_QUERY`` query tokens (bfloat16 and float16) are cut into query tiles of
-    ``64 // G`` tokens for the MFMA prefill kernel, which reads each key and value row once per
+    ``128 // G`` tokens for the MFMA prefill kernel, which reads each key and value row once per
     tile; the other query tokens go to the per-token kernel.
 """
 from __future__ import annotations
@@ -243,8 +243,9 @@ def paged_attention_hip(query, k_cache, v_cache, block_tables, seq_lens, query_s
     allocated per call, resp. taken from this module's per-device, per-stream buffer, when not
     given.  ``max_query_len``: an upper bound of ``query_lens`` (1 for a decode step, which then
     takes the per-token kernel without reading the batch layout on the host).  ``plan``: a
-    ``PagedAttentionPlan`` of this batch layout (then nothing is read on the host).  ``stream``: a ``torch.cuda.Stream`` or a raw HIP stream handle, default the current
-    stream; the call's own temporaries are made on it, so nothing orders them against another.
+    ``PagedAttentionPlan`` of this batch layout (then nothing is read on the host).  ``stream``: a
+    ``torch.cuda.Stream`` or a raw HIP stream handle, default the current stream; the call's own temporaries
+    are made on it, so nothing orders them against another.
     """
     import torch
 
