@@ -290,9 +290,9 @@ def test_plan_reused_across_layers_and_refused_for_another_layout(device):
 
 
 @pytest.mark.parametrize("d", [128, 64])
-def test_prefill_tile_merged_from_many_partitions(device, d):
-    # one tile over 9000 positions splits into more partitions than the merge's LDS weight table
-    # holds (the one-pass rescaled merge) and a 4000-position tile into fewer (the table)
+def test_prefill_tile_merged_from_many_segments(device, d):
+    # one tile over 9000 positions is cut between many workgroups, one over 4000 between fewer; the last
+    # to arrive merges the segments one after the other
     case = make_case(97 + d, [9000, 4000], [20, 30], d=d)
     check(case, device)
 
