@@ -17,8 +17,8 @@
  * scores, their sums and the accumulators are float32, and a softmax weight w (relative to its
  * column's largest) enters the value product as two 16-bit parts: to 2^-17 w in bfloat16, to 2^-22 w
  * + 2^-49 (prefill tiles: 2^-38) in float16.  An infinite value in a visible row gives infinity, except
- * in a prefill tile, whose outputs are NaN in that dim for the tokens that see it and for those
- * up to 63 positions before it.
+ * in a prefill tile, whose outputs are NaN in that dim for the tokens that see it and for the tile's
+ * tokens before it.
  *
  * Layouts: query/out (total_q, num_heads_q, head_dim), caches (num_blocks, block_size,
  * num_kv_heads, head_dim), each with arbitrary element strides except a unit head_dim stride and
