@@ -41,7 +41,7 @@ constexpr int kMinPart = 64;
 // partitions of a row merged through a table of their weights in LDS (one long row of few KV heads has
 // hundreds): the loop that takes more reads three words per partition and output one after the other.
 // one row of 17000 .. 65536 positions, 1 .. 3 KV heads (266 .. 1024 partitions, bf16, head_dim 128,
-// G = 1 .. 8): 29-296 us with the table, 75-1145 by the loop
+// G = 1 .. 8): 18-121 us with the table, 75-1145 by the loop
 constexpr int kMaxMerge = 1024;
 // workgroups a launch aims for before splitting stops: four per CU (the 128-dim 16-bit kernels hold three at once)
 constexpr int kTargetGroups = 1024;
@@ -83,6 +83,8 @@ struct PaParams {
 // ---- element loads / stores -------------------------------------------------------------------
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <int N> struct Int { static constexpr int value = N; };
 
 struct Bf16 {};
 struct F16 {};
@@ -353,8 +355,20 @@ __device__ __forceinline__ void finish_partition(const PaParams& p, int qi, int 
       const int h = kvh * G + g;
       const int64_t base = ((int64_t)qi * p.hq + h) * p.max_parts;
       float o = 0.f;
-#pragma unroll 4
-      for (int i = 0; i < arrivals; ++i) o = fmaf(s_w[g * kMaxMerge + i], ld_dev(&p.ws_acc[(base + i) * D + d]), o);
+      int i = 0;
+      // so many partitions, their loads in flight together: 8, then 4, then one by one (1 x 65,536, 8 heads on 1
+      // KV head: 284 us with 4 and one by one, 121 so; 8 x 300, five partitions: 10.6 both)
+      auto add = [&](auto count) {
+        float a[decltype(count)::value];
+#pragma unroll
+        for (int j = 0; j < decltype(count)::value; ++j) a[j] = ld_dev(&p.ws_acc[(base + i + j) * D + d]);
+#pragma unroll
+        for (int j = 0; j < decltype(count)::value; ++j) o = fmaf(s_w[g * kMaxMerge + i + j], a[j], o);
+        i += decltype(count)::value;
+      };
+      while (i + 8 <= arrivals) add(Int<8>{});
+      if (i + 4 <= arrivals) add(Int<4>{});
+      while (i < arrivals) add(Int<1>{});
       const float l = s_l[g];
       store_one<T>(p.out, (int64_t)qi * p.so_tok + (int64_t)h * p.so_head + d, l > 0.f ? o / l : 0.f);
     }
