@@ -679,11 +679,11 @@ __device__ __forceinline__ void plain_partition(const PaParams& p, int qi, int k
 //     write and the 8 rows of a transposing read over the 64 banks (the counters show 20 conflict
 //     cycles left in a step, of some thousands).
 // Bound by HBM.  Measured (bf16, 8 KV heads of 128 dims, blocks of 16; the vector form, then this):
-// 8 x 8192 at G = 3: 60 -> 58 us; 64 x 2048: 108 -> 108 (5.0 TB/s); 256 x 512: 107 -> 98; G = 4, 64 x 2048:
-// 141 -> 108; G = 8, 64 x 2048: 310 -> 113.  G = 1 gains least: one row of 64 to 8 of 300 positions 5-12%
-// faster, 8 x 2048 20.2 -> 20.9, 64 x 2048 of 64 dims 47 -> 50.  At 128 dims three waves a SIMD (138 to 150
-// registers of 168): four spill 8 bytes and measured 63 us at 8 x 8192, 111 at 64 x 2048 and 63 at 256 rows
-// of up to 512, two 61, 103 and 60, three 58, 107 and 57.
+// 8 x 8192 at G = 3: 60 -> 56 us; 64 x 2048: 108 -> 107 (5.0 TB/s); 256 x 512: 107 -> 98; G = 4, 64 x 2048:
+// 141 -> 109; G = 8, 64 x 2048: 310 -> 109.  G = 1 gains least: 8 x 2048 20.2 -> 19.1, 64 x 2048 of 64 dims 57
+// both (47 -> 50 where the last-level cache holds most of it).  At 128 dims three waves a SIMD (159 to 168
+// registers of 168): four spill, and an earlier form took 63 us with them at 8 x 8192, 111 at 64 x 2048 and 63
+// at 256 rows of up to 512, with two 61, 103 and 60, with three 58, 107 and 57.
 // BW as in the prefill kernel: a row's address is a scalar plus a lane's fixed offset.
 template <typename T, int D, int G, bool BW>
 __global__ __launch_bounds__(kThreads)
@@ -834,21 +834,23 @@ __global__ __launch_bounds__(kThreads)
     load_v();
     __builtin_amdgcn_sched_barrier(0);
   }
-  for (; base < n; base += kWaves * kStep) {
+  // one step; `more`: the next step's rows are requested before the arithmetic, loads without a branch
+  // around them, so that the wait for the older ones leaves them in flight
+  auto step = [&](auto more) {
     const uint32_t okw = ok;
     store_rows(sk, kreg);
-    // the next step's rows, past the end the last ones again: loads without a branch around them, so
-    // that the wait for the older ones leaves them in flight
-    place_rows(base + kWaves * kStep);
-    load_k();
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (decltype(more)::value != 0) {
+      place_rows(base + kWaves * kStep);
+      load_k();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (okw != kAllOk) {   // weight 0 times a row not of this sequence must be 0
 #pragma unroll
       for (int i = 0; i < NL; ++i)
         if (!((okw >> (RPI * i + row0)) & 1u)) vreg[i] = u32x4{0u, 0u, 0u, 0u};
     }
     store_rows(sv, vreg);
-    load_v();
+    if constexpr (decltype(more)::value != 0) load_v();
     __builtin_amdgcn_wave_barrier();   // the wave's own LDS rows: in order, no workgroup barrier
     // S^T = K Q^T
     f32x4_t st[NB];
@@ -929,7 +931,11 @@ __global__ __launch_bounds__(kThreads)
       }
     }
     __builtin_amdgcn_wave_barrier();
-  }
+  };
+  for (; base + kWaves * kStep < n; base += kWaves * kStep) step(Int<1>{});
+  // the wave's last step requests none (it is one of one or two where partitions are 64 or 128 positions: 8 x 2048
+  // at G = 1 20.0 us with its rows requested again, 19.1 without)
+  if (base < n) step(Int<0>{});
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
 
